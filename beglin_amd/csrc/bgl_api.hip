@@ -886,6 +886,7 @@ static bool qm_ok(bgl_ctx *c, int kind, int K) {
 
 static int run_gemv_q(bgl_ctx *c, int n, const BglDevTensor *Ts, const float *x_dev, int M, const float *const *bias,
                       float *const *y) {
+    if (gemm_q_ok(c, Ts, n, M)) return run_gemm_q(c, n, Ts, x_dev, c->prep_u, c->prep_h, M, bias, y);
     // 5..16 columns: the matrix-core kernel (one MFMA column per activation column), where its
     // terms (and, quantizing in the kernel, the columns' codes) fit LDS.  (Qwen2.5-1.5B g256sf cfg2
     // step: 8 columns 1.239 -> 1.115 ms; at 4 columns the dot4 kernel stays ahead, 0.957 against
@@ -983,7 +984,7 @@ int run_down_swiglu_w4a8(bgl_ctx *c, const BglDevTensor &down, const float *g, c
     const int mbmax = q_mb_max(kind, K);
     if (mbmax < 2) return 1;
     const int passes = std::min(M, mbmax) * ((K + 255) / 256);
-    if (!(c->q_prep == 1 || (c->q_prep < 0 && passes >= BGL_Q_PREP_MIN_PASSES))) return 1;
+    if (!gemm_q_ok(c, &down, 1, M) && !(c->q_prep == 1 || (c->q_prep < 0 && passes >= BGL_Q_PREP_MIN_PASSES))) return 1;
     c->prep_u = u;
     c->prep_h = h;
     const float *nob[1] = {nullptr};

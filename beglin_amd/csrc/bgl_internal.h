@@ -100,6 +100,10 @@ int run_gemm_mfma(bgl_ctx *c, int n, const BglDevTensor *Ts, const float *x_dev,
                   float *const *y, const int *ystride, float *glu_h = nullptr);
 // The dense MLP block at one W4A8 column in one launch (bgl_mlp_q.hip): the formats it takes, and the call.
 int run_down_swiglu_w4a8(bgl_ctx *c, const BglDevTensor &down, const float *g, const float *u, float *h, int M, float *y);
+// W4A8 products of more than 16 columns (bgl_gemm_q.hip): the calls it takes, and the call.
+bool gemm_q_ok(bgl_ctx *c, const BglDevTensor *Ts, int n, int M);
+int run_gemm_q(bgl_ctx *c, int n, const BglDevTensor *Ts, const float *x_dev, const float *u, float *h, int M,
+               const float *const *bias, float *const *y);
 bool mlp_q_ok(bgl_ctx *c, const BglDevTensor &gate, const BglDevTensor &up, const BglDevTensor &down);
 int run_mlp_q(bgl_ctx *c, const BglDevTensor &gate, const BglDevTensor &up, const BglDevTensor &down, const float *x,
               float *h, float *y);
