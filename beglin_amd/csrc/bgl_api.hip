@@ -1023,11 +1023,7 @@ extern "C" int bgl_matmul_group_dev(bgl_ctx *c, int n, const bgl_tensor *const *
         return bgl_fail(BGL_E_UNSUPPORTED, "kind %d has fp32-activation kernels only", kind);
     HIPCHK(hipSetDevice(c->device));
     if (act == BGL_ACT_W4A8 && fused_q_ok(c, kind, Ts[0].K, M)) return run_gemv_q(c, n, Ts, x_dev, M, bias_dev, y_dev);
-    if (act == BGL_ACT_F32 && M >= BGL_MFMA_MIN_M && !c->no_mfma) {
-        bool ok = true;
-        for (int i = 0; i < n; i++) ok = ok && bgl_mfma_ok(Ts[i].fmt, Ts[i].bits);
-        if (ok) return run_gemm_mfma(c, n, Ts, x_dev, M, bias_dev, y_dev, nullptr);
-    }
+    if (act == BGL_ACT_F32 && mfma_takes(c, n, Ts, M)) return run_gemm_mfma(c, n, Ts, x_dev, M, bias_dev, y_dev, nullptr);
     // one fp32 column over a short K: the GEMV makes the activation digits itself (no prep launch)
     if (act == BGL_ACT_F32 && M == 1 && !c->no_gemv_x && gemv_x_kind(kind) &&
         (c->x_fuse == 1 || (c->x_fuse < 0 && Ts[0].K <= BGL_GEMV_X_FUSE_MAX_K))) {

@@ -27,7 +27,7 @@ struct bgl_ctx {
     bool own_stream = false;
     int max_waves = 16;                   // wavefronts per GEMV workgroup cap (BGL_MAX_WAVES)
     bool no_fused = false;                // BGL_NO_FUSED_Q=1: W4A8 M=1 through the separate prep kernel
-    bool no_mfma = false;                 // BGL_NO_MFMA=1: fp32-activation M >= 16 through the dot4 kernels
+    bool no_mfma = false;                 // BGL_NO_MFMA=1: several fp32-activation columns through the dot4 kernels
     int min_blocks = 256;                 // fused W4A8: split tiles until at least this many workgroups
     float mf_pcap = 1.0f;                 // matrix-core K split: partials (written + read) at most this x the weight bytes
     int force_tr = 0;                     // BGL_FORCE_TR: fixed rows per workgroup (tuning)
@@ -92,8 +92,10 @@ int pick_waves(bgl_ctx *c, int nunits);
 int run_gemv(bgl_ctx *c, int n, const BglDevTensor *Ts, int act, const GemvAct &A, int M,
              const float *const *bias, float *const *y, const int *ystride);
 // Batched fp32-activation GEMM on the matrix cores (bgl_mfma.hip): formats it takes, and the call.
-#define BGL_MFMA_MIN_M 16
+#define BGL_MFMA_MIN_M 16               // the routed FFN's shared experts leave the gather from this many tokens
 bool bgl_mfma_ok(int fmt, int bits);
+// Whether a group's products of M fp32 columns run there.
+bool mfma_takes(const bgl_ctx *c, int n, const BglDevTensor *Ts, int M);
 // glu_h (n == 2, a gate/up pair of one shape): the reduce launch also forms h = silu(gate) * up
 // into glu_h [M][N] (k_swiglu's arithmetic), so the caller needs no SwiGLU launch.
 int run_gemm_mfma(bgl_ctx *c, int n, const BglDevTensor *Ts, const float *x_dev, int M, const float *const *bias,

@@ -1,4 +1,4 @@
-// bgl_mfma.hip -- batched GEMM for M >= 16 activation rows on the gfx950 fp16 matrix cores
+// bgl_mfma.hip -- batched GEMM for M >= 2 activation rows on the gfx950 fp16 matrix cores
 // (the M-column case of gemm_qXg64_mt / qng64_matmul_f32, q4gemv.h:761-769, qng64_dense.c:70-79).
 //
 // Numerics.  Weight codes are exact in fp16 (int4 and int8 codes, qNg64 codes for n <= 10), so
@@ -42,6 +42,8 @@
 // of a 14336 x 4096 tensor at M = 32 took 3.8 us to write that way; staged, every lane writes 16
 // consecutive bytes and each wave 1 KB runs (2 us faster per such launch).
 #include <string.h>
+
+#include <algorithm>
 
 #include "bgl_gemv_impl.h"
 #include "bgl_internal.h"
@@ -834,8 +836,87 @@ static double mf_weight_bytes(const BglDevTensor &T) {
     return per * T.N * T.K;
 }
 
+// A split's K range must fit the workgroup's LDS (kpm steps); beyond that, split K until
+// the grid has ~min_blocks workgroups while the partials (written and read back once
+// each) stay under mf_pcap x the weight bytes (1 by default: at 0.5 the 4096 x 4096
+// qNg64 n=5 tensors of a 32-column launch ran 64 workgroups, 19.3 us, against 128 and
+// 15.0 us; finer splits than 16 K-steps measured no faster).
+static int mf_splits(const bgl_ctx *c, const BglDevTensor &T, int Mc, int &kps) {
+    const int CT = (Mc + 15) / 16, KS = T.K / 32, wgr = (T.ntiles + MF_TILES - 1) / MF_TILES;
+    const int kpm = CT == 1 ? mf_kps_max(1) : CT == 2 ? mf_kps_max(2) : CT == 3 ? mf_kps_max(3) : mf_kps_max(4);
+    const int smin = (KS + kpm - 1) / kpm;
+    int S = (c->min_blocks + wgr - 1) / wgr;
+    const int capS = (int)(c->mf_pcap * mf_weight_bytes(T) / (8.0 * Mc * T.N));
+    if (S > capS) S = capS;
+    if (S < smin) S = smin;
+    if (S < 1) S = 1;
+    kps = (KS + S - 1) / S;
+    kps = (kps + MF_KSTEP_PAD - 1) / MF_KSTEP_PAD * MF_KSTEP_PAD;
+    if (kps > kpm) kps = kpm;
+    return (KS + kps - 1) / kps;
+}
+
+// The K-split partials (floats) of a launch of Mc columns.
+static size_t mf_partials(const bgl_ctx *c, int n, const BglDevTensor *Ts, int Mc) {
+    size_t fl = 0;
+    for (int i = 0; i < n; i++) {
+        int kps;
+        const int S = mf_splits(c, Ts[i], Mc, kps);
+        if (S > 1) fl += (size_t)S * Mc * Ts[i].N;
+    }
+    return fl;
+}
+
+// Scratch for the same call at fewer columns, which a caller may capture once this one has run: the
+// partials do not grow strictly with the columns (this bounds them), and the fewest columns take the
+// digits of k_act_x24.
+static int mf_reserve_fewer(bgl_ctx *c, int n, const BglDevTensor *Ts, int M) {
+    const int Mc = std::min(M, 16 * MF_MAXCT), CT = (Mc + 15) / 16;
+    const int kpm = CT == 1 ? mf_kps_max(1) : CT == 2 ? mf_kps_max(2) : CT == 3 ? mf_kps_max(3) : mf_kps_max(4);
+    const size_t ng = Ts[0].K / 64, md = std::min(M, 4);
+    double fl = 0.0;
+    for (int i = 0; i < n; i++) {
+        const int wgr = (Ts[i].ntiles + MF_TILES - 1) / MF_TILES, smin = (Ts[i].K / 32 + kpm - 1) / kpm;
+        const double most = std::min((double)((c->min_blocks + wgr - 1) / wgr) * Mc * Ts[i].N, c->mf_pcap * mf_weight_bytes(Ts[i]) / 8.0);
+        fl += std::max(most, smin > 1 ? (double)smin * Mc * Ts[i].N : 0.0);
+    }
+    const size_t pb = (size_t)fl * 4, db = 2 * md * ng * 192;
+    // operands that bgl_prep_act_dev left stay where they are
+    const bool dig = !c->prep_reuse;
+    if (c->part.bytes >= pb && (!dig || (c->act_w.bytes >= db && c->act_s.bytes >= 2 * md * ng * 4 && c->act_sum.bytes >= 4 * md * ng * 16))) return 0;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    HIPCHK(hipStreamIsCapturing(c->stream, &cs));
+    if (cs != hipStreamCaptureStatusNone) return 0;                // this call may still have all that it needs
+    if (dbuf_reserve(c, c->part, pb, false)) return bgl_last_code();
+    if (dig && (dbuf_reserve(c, c->act_w, db, false) || dbuf_reserve(c, c->act_s, 2 * md * ng * 4, false) ||
+                dbuf_reserve(c, c->act_sum, 4 * md * ng * 16, false)))
+        return bgl_last_code();
+    return 0;
+}
+
+// From 2 columns.  The dot4 kernels multiply three digits per value and column (k_gemv: 4 or 8 columns
+// a launch), the matrix cores take 16 columns for the price of one; a wave's weights are the same.
+// Measured, us, dot4 / here: q4g64 28672 x 4096 at 2 / 5 / 15 columns 40.2 / 28.9, 73.1 / 29.4, 153 /
+// 32.5; 4096 x 4096 14.3 / 12.3, 19.7 / 12.4, 35.8 / 13.0; 1536 x 1536 13.6 / 11.3, 17.5 / 11.7, 31.8 /
+// 12.4; q8g64 28672 x 4096 at 2 columns 41.1 / 34.9; qNg64 n = 6, 10 at 2: 54.5 / 38.8, 56.8 / 47.7.
+// qNg64 n <= 3 reads its crumbs and bits a dword at a time here: n = 3 at 2 / 4 / 8 columns 49.4 / 52.7,
+// 52.4 / 53.0, 94.1 / 53.3.  Against 64 bits the N(0, 1) products err by 1.6e-7 here, 2.9e-7 there.
+// Below 16 columns the dot4 kernels also keep what they alone can run: tensors of 2 GiB and more, and
+// no-alloc calls whose K-split partials do not fit the fixed array.
+bool mfma_takes(const bgl_ctx *c, int n, const BglDevTensor *Ts, int M) {
+    if (c->no_mfma || M < 2) return false;
+    for (int i = 0; i < n; i++)
+        if (!bgl_mfma_ok(Ts[i].fmt, Ts[i].bits)) return false;
+    if (M >= 16) return true;
+    for (int i = 0; i < n; i++)
+        if ((double)Ts[i].ntiles * Ts[i].cpr * 1024.0 >= 2147483648.0) return false;
+    if (c->fixed_base && c->fixed_used + mf_partials(c, n, Ts, M) * 4 + 256 > c->fixed_cap) return false;
+    return M >= (Ts[0].fmt == BGL_QNG64 && Ts[0].bits <= 3 ? 5 : 2);
+}
+
+
 // y[m][n] = bias[n] + sum_k W[n][k] x[m][k] for the n tensors of a group sharing x (same format,
-// width and K), M >= 1 columns (the caller routes M >= 16 here).  Columns go in launches of up to
+// width and K), M >= 1 columns (mfma_takes says which calls come here).  Columns go in launches of up to
 // 64: one fragment prep, one GEMM over every tensor, and one reduce when any tensor splits K.
 int run_gemm_mfma(bgl_ctx *c, int n, const BglDevTensor *Ts, const float *x_dev, int M, const float *const *bias,
                   float *const *y, const int *ystride, float *glu_h) {
@@ -851,7 +932,10 @@ int run_gemm_mfma(bgl_ctx *c, int n, const BglDevTensor *Ts, const float *x_dev,
         const double wb = (double)Ts[i].ntiles * Ts[i].cpr * 1024.0;
         if (wb >= 2147483648.0) return bgl_fail(BGL_E_UNSUPPORTED, "MFMA path: tensor %d holds >= 2 GiB (32-bit buffer offsets)", i);
     }
-    const int KS = K / 32;
+    if (!c->fixed_base) {
+        const int rc = mf_reserve_fewer(c, n, Ts, M);
+        if (rc) return rc;
+    }
     // The chunks run in stream order, so each reuses the same K-split partials.  In a no-alloc call
     // the fixed array is handed out by a bump pointer: rewind it to this mark before every chunk,
     // so the first (largest) chunk's reservation bounds the whole call.
@@ -860,7 +944,6 @@ int run_gemm_mfma(bgl_ctx *c, int n, const BglDevTensor *Ts, const float *x_dev,
         const int Mc = M - m0 < 16 * MF_MAXCT ? M - m0 : 16 * MF_MAXCT;
         if (c->fixed_base) c->fixed_used = fixed_mark;
         const int CT = (Mc + 15) / 16;
-        const int kpm = CT == 1 ? mf_kps_max(1) : CT == 2 ? mf_kps_max(2) : CT == 3 ? mf_kps_max(3) : mf_kps_max(4);
         MfmaLaunch L;
         memset(&L, 0, sizeof L);
         L.ntasks = n; L.M = Mc; L.x = x_dev + (size_t)m0 * K;
@@ -870,21 +953,8 @@ int run_gemm_mfma(bgl_ctx *c, int n, const BglDevTensor *Ts, const float *x_dev,
         for (int i = 0; i < n; i++) {
             const BglDevTensor &T = Ts[i];
             const int wgr = (T.ntiles + MF_TILES - 1) / MF_TILES;
-            // A split's K range must fit the workgroup's LDS (kpm steps); beyond that, split K until
-            // the grid has ~min_blocks workgroups while the partials (written and read back once
-            // each) stay under mf_pcap x the weight bytes (1 by default: at 0.5 the 4096 x 4096
-            // qNg64 n=5 tensors of a 32-column launch ran 64 workgroups, 19.3 us, against 128 and
-            // 15.0 us; finer splits than 16 K-steps measured no faster).
-            const int smin = (KS + kpm - 1) / kpm;
-            int S = (c->min_blocks + wgr - 1) / wgr;
-            const int capS = (int)(c->mf_pcap * mf_weight_bytes(T) / (8.0 * Mc * T.N));
-            if (S > capS) S = capS;
-            if (S < smin) S = smin;
-            if (S < 1) S = 1;
-            int kps = (KS + S - 1) / S;
-            kps = (kps + MF_KSTEP_PAD - 1) / MF_KSTEP_PAD * MF_KSTEP_PAD;
-            if (kps > kpm) kps = kpm;
-            S = (KS + kps - 1) / kps;
+            int kps;
+            const int S = mf_splits(c, T, Mc, kps);
             S_[i] = S;
             MfmaTask &t = L.t[i];
             t.T = T; t.bias = bias ? bias[i] : nullptr;

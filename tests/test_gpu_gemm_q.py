@@ -55,6 +55,7 @@ def run(ctx, torch, kind, packed, x, biases, shapes, bits_equal_to):
     xd = torch.from_numpy(x).cuda()
     ys = [torch.full((x.shape[0], o), float("nan"), device="cuda") for o in shapes]
     bd = [torch.from_numpy(b).cuda() if b is not None else None for b in biases]
+    torch.cuda.synchronize()
     ctx.matmul_group(ts, xd, ys, act=1, biases=bd)
     ctx.sync()
     for t, y, r in zip(ts, ys, bits_equal_to):
@@ -108,7 +109,10 @@ def test_gemm_q_weight_scales_at_the_ends_of_fp32(ctx, torch_dev, oracle, kind, 
         ref = oracle.matmul_sdot(kind, pk, sc, x, sub=sub)
     t = ctx.bind(kind, pk, sc, out, inn, sub=sub)
     y = torch_dev.empty((M, out), device="cuda")
-    ctx.matmul(t, torch_dev.from_numpy(x).cuda(), y, act=1)
+    xd = torch_dev.from_numpy(x).cuda()
+    torch_dev.cuda.synchronize()
+    ctx.matmul(t, xd, y, act=1)
+    ctx.sync()
     got = y.cpu().numpy()
     t.free()
     assert np.array_equal(np.isnan(got), np.isnan(ref))
@@ -128,7 +132,10 @@ def test_gemm_q_mlp_block(ctx, torch_dev, oracle, kind, M):
     ref = oracle.matmul_sdot(kind, ws[2][0], ws[2][1], h, sub=ws[2][2])
     ts = [ctx.bind(kind, p, s, p.shape[0], k, sub=sub) for (p, s, sub), k in zip(ws, (H, H, I))]
     y, hd = torch_dev.empty((M, H), device="cuda"), torch_dev.empty((M, I), device="cuda")
-    ctx.mlp(*ts, torch_dev.from_numpy(x).cuda(), y, act=1, h_dev=hd)
+    xd = torch_dev.from_numpy(x).cuda()
+    torch_dev.cuda.synchronize()
+    ctx.mlp(*ts, xd, y, act=1, h_dev=hd)
+    ctx.sync()
     assert np.array_equal(hd.cpu().numpy().view(np.uint32), h.view(np.uint32))
     assert np.array_equal(y.cpu().numpy().view(np.uint32), ref.view(np.uint32))
     for t in ts:

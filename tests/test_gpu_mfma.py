@@ -268,3 +268,57 @@ def test_mfma_tiny_and_huge_columns(ctx, torch_dev, oracle, kind, bits):
     # outputs ~1e-41 are subnormal (spacing 2^-149): a few spacings of absolute error
     assert np.max(np.abs(got[2].astype(np.float64) - ref[2])) <= 16 * 2.0 ** -149
     assert np.max(np.abs(ref[2])) > 0.0 and np.all(got[4] == 0.0)
+
+
+@pytest.mark.parametrize("kind,bits", [(1, 0), (5, 0), (2, 0), (4, 2), (4, 3), (4, 7), (4, 10)])
+def test_mfma_few_columns(ctx, torch_dev, oracle, kind, bits):
+    """2..15 columns: K of one group, around a K split's 16 steps and past it (odd groups, an odd
+    pair of qNg64), rows that leave tiles partly filled."""
+    torch = torch_dev
+    for out, inn in ((70, 64), (300, 576), (130, 4160)):
+        w = weights(300 + kind + bits + inn, out, inn)
+        p, s = quant(oracle, kind, w, bits)
+        t = ctx.bind(kind, p, s, out, inn, bits=bits)
+        for M in (2, 3, 5, 15):
+            say("few columns", kind, bits, out, inn, M)
+            x = seeded_normal(310 + M, (M, inn))
+            xd, y = torch.from_numpy(x).cuda(), torch.full((M, out), float("nan"), device="cuda")
+            torch.cuda.synchronize()
+            ctx.matmul(t, xd, y)
+            ctx.sync()
+            assert relerr(y.cpu().numpy(), oracle.gemm_f32(kind, p, s, x, bits=bits)) <= TOL
+        t.free()
+
+
+def test_mfma_call_sizes_scratch_for_fewer_columns(torch_dev, oracle):
+    """A call of 15 columns outside a capture is enough for captures of the same product at 7, 3 and 1
+    columns (K split differently, digits instead)."""
+    import beglin_amd
+    torch = torch_dev
+    st = torch.cuda.Stream()
+    c = beglin_amd.Context(0, st.cuda_stream)
+    out, inn = 256, 8192
+    w = weights(77, out, inn)
+    p, s = oracle.quantize_q4g64(w)
+    t = c.bind(1, p, s, out, inn)
+    x = torch.from_numpy(seeded_normal(78, (15, inn))).cuda()
+    y = torch.empty((15, out), device="cuda")
+    torch.cuda.synchronize()
+    c.matmul(t, x, y)
+    c.sync()
+    ref = oracle.gemm_f32(1, p, s, x.cpu().numpy())
+    for M in (7, 3, 1):
+        say("fewer columns captured", M)
+        xm, ym = x[:M].contiguous(), torch.empty((M, out), device="cuda")
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=st):
+            c.matmul(t, xm, ym)
+        for _ in range(2):
+            ym.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert relerr(ym.cpu().numpy(), ref[:M]) <= TOL
+        del g
+    t.free()
+    c.close()
