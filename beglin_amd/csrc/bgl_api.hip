@@ -403,7 +403,7 @@ static int repack_into(bgl_ctx *c, int kind, int bits, int out, int in, const vo
                            in * (kind == BGL_F16 ? 2 : kind == BGL_F32 ? 4 : 1), (uint8_t *)w);
         break;
     case BGL_QNG64:
-        hipLaunchKernelGGL(k_repack_qng, dim3(nblk(rows * T.nunits, 64)), dim3(64), 0, c->stream, (const uint8_t *)dpk, out, in, bits, (uint8_t *)w);
+        bgl_repack_qng((const uint8_t *)dpk, out, in, bits, (uint8_t *)w, c->stream);
         break;
     }
     long nu = rows * T.nunits;
@@ -592,20 +592,20 @@ extern "C" int bgl_quantize_dev(bgl_ctx *c, int kind, int bits, int qng64_encode
     switch (kind) {
     case BGL_Q4G64:
         units = (long)out * (in / 64);
-        hipLaunchKernelGGL(k_quant_q4g64, dim3(nblk(units)), dim3(256), 0, c->stream, w_dev, out, in, (uint8_t *)dpk, (float *)dsc);
+        hipLaunchKernelGGL(k_quant_q4g64, dim3(nblk(units, PK_THREADS)), dim3(PK_THREADS), 0, c->stream, w_dev, out, in, (uint8_t *)dpk, (float *)dsc);
         break;
     case BGL_Q8G64:
         units = (long)out * (in / 64);
-        hipLaunchKernelGGL(k_quant_q8g64, dim3(nblk(units)), dim3(256), 0, c->stream, w_dev, out, in, (int8_t *)dpk, (float *)dsc);
+        hipLaunchKernelGGL(k_quant_q8g64, dim3(nblk(units, PK_THREADS)), dim3(PK_THREADS), 0, c->stream, w_dev, out, in, (int8_t *)dpk, (float *)dsc);
         break;
     case BGL_QNG64:
         units = (long)out * (in / 64);
-        hipLaunchKernelGGL(k_quant_qng64, dim3(nblk(units, 64)), dim3(64), 0, c->stream, w_dev, out, in, bits, qng64_encoder ? 1 : 0,
+        hipLaunchKernelGGL(k_quant_qng64, dim3(nblk(units, PK_THREADS)), dim3(PK_THREADS), 0, c->stream, w_dev, out, in, bits, qng64_encoder ? 1 : 0,
                            (uint8_t *)dpk, (float *)dsc);
         break;
     case BGL_Q4G32H:
         units = (long)out * (in / 32);
-        hipLaunchKernelGGL(k_quant_q4g32h, dim3(nblk(units)), dim3(256), 0, c->stream, w_dev, out, in, (uint8_t *)dpk, (uint16_t *)dsc);
+        hipLaunchKernelGGL(k_quant_q4g32h, dim3(nblk(units, PK_THREADS)), dim3(PK_THREADS), 0, c->stream, w_dev, out, in, (uint8_t *)dpk, (uint16_t *)dsc);
         break;
     case BGL_Q4G256SF:
         units = (long)out * (in / 256);
@@ -655,7 +655,7 @@ extern "C" int bgl_tensor_info(const bgl_tensor *t, int *kind, int *bits, int *o
 extern "C" int bgl_dequant_dev(bgl_ctx *c, const bgl_tensor *t, int row0, int nrows, float *out_dev) {
     if (!c || !t || !out_dev || !t->experts.empty()) return bgl_fail(BGL_E_ARG, "bgl_dequant_dev: bad argument");
     if (row0 < 0 || nrows <= 0 || row0 + nrows > t->T.N) return bgl_fail(BGL_E_ARG, "bgl_dequant_dev: rows out of range");
-    hipLaunchKernelGGL(k_dequant, dim3(nblk((long)nrows * t->T.K)), dim3(256), 0, c->stream, t->T, row0, nrows, out_dev);
+    hipLaunchKernelGGL(k_dequant, dim3((unsigned)((long)(t->T.K / 64) * ((nrows + 15) / 16))), dim3(256), 0, c->stream, t->T, row0, nrows, out_dev);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -685,8 +685,9 @@ int prep_act(bgl_ctx *c, int act, int gq, const float *x_dev, int M, int K, Gemv
             return bgl_last_code();
         int tok = prof_begin(c, 0);
         hipLaunchKernelGGL(k_act_x24, dim3(nblk((long)M * ng * 64)), dim3(256), 0, c->stream, x_dev, M, K,
-                           (int8_t *)c->act_w.p, (float *)c->act_s.p, (int *)c->act_sum.p);
+                           (int8_t *)c->act_w.p, (float *)c->act_s.p, (int *)c->act_sum.p, c->prep_u, c->prep_h);
         prof_end(c, tok);
+        if (c->prep_h) x_dev = c->prep_h;      // the columns just formed: the non-finite slow path reads them
     } else {
         if (dbuf_reserve(c, c->act_w, (size_t)M * K, false) || dbuf_reserve(c, c->act_s, (size_t)M * (K / gq) * 4, false) ||
             dbuf_reserve(c, c->act_sum, (size_t)M * (K / 64) * 4, false))
@@ -990,6 +991,21 @@ int run_down_swiglu_w4a8(bgl_ctx *c, const BglDevTensor &down, const float *g, c
     const float *nob[1] = {nullptr};
     float *ys[1] = {y};
     const int rc = run_gemv_q(c, 1, &down, g, M, nob, ys);
+    c->prep_u = nullptr;
+    c->prep_h = nullptr;
+    return rc;
+}
+
+// The same at fp32 activations, where the down projection multiplies prepared digits (one column over a
+// long K, and the formats the matrix cores do not take): k_act_x24 forms h, no SwiGLU launch.  (Llama-8B
+// qNg64 n=6 block at one column 46.9 -> 44.9 us.)  Returns 1 (nothing launched) elsewhere.
+int run_down_swiglu_f32(bgl_ctx *c, const bgl_tensor *down, const float *g, const float *u, float *h, int M, float *y) {
+    const BglDevTensor &T = down->T;
+    if (mfma_takes(c, 1, &T, M) || !(gemv_x_kind(T.fmt))) return 1;
+    if (M == 1 && !c->no_gemv_x && (c->x_fuse == 1 || (c->x_fuse < 0 && T.K <= BGL_GEMV_X_FUSE_MAX_K))) return 1;
+    c->prep_u = u;
+    c->prep_h = h;
+    const int rc = bgl_matmul_dev(c, down, BGL_ACT_F32, g, nullptr, y, M);
     c->prep_u = nullptr;
     c->prep_h = nullptr;
     return rc;

@@ -41,7 +41,7 @@ struct bgl_ctx {
     DevBuf act_w, act_s, act_sum;         // activation operands of the current call
     int prep_act = -1, prep_gq = 0, prep_M = 0, prep_K = 0;   // what act_* currently hold
     const float *prep_x = nullptr;        // the raw fp32 columns they were made from (non-finite slow path)
-    const float *prep_u = nullptr;        // set around run_down_swiglu_w4a8: the prep launch forms h = SwiGLU(x, prep_u)
+    const float *prep_u = nullptr;        // set around run_down_swiglu_*: the prep launch forms h = SwiGLU(x, prep_u)
     float *prep_h = nullptr;              //   into prep_h
     bool prep_reuse = false;              // act_* come from bgl_prep_act_dev (or a host drop-in): bgl_matmul_prepped_dev may use them
     DevBuf prep_xc;                       // bgl_prep_act_dev's own copy of the fp32 columns (prep_x points here)
@@ -106,6 +106,7 @@ int run_down_swiglu_w4a8(bgl_ctx *c, const BglDevTensor &down, const float *g, c
 bool gemm_q_ok(bgl_ctx *c, const BglDevTensor *Ts, int n, int M);
 int run_gemm_q(bgl_ctx *c, int n, const BglDevTensor *Ts, const float *x_dev, const float *u, float *h, int M,
                const float *const *bias, float *const *y);
+int run_down_swiglu_f32(bgl_ctx *c, const bgl_tensor *down, const float *g, const float *u, float *h, int M, float *y);
 bool mlp_q_ok(bgl_ctx *c, const BglDevTensor &gate, const BglDevTensor &up, const BglDevTensor &down);
 int run_mlp_q(bgl_ctx *c, const BglDevTensor &gate, const BglDevTensor &up, const BglDevTensor &down, const float *x,
               float *h, float *y);

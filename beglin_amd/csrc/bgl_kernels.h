@@ -203,9 +203,10 @@ struct MoeTask {
 };
 
 // ---- kernels (bgl_prep.hip) ----
+#define PK_THREADS 128           // threads of a packer's workgroup (its groups of 64 take 33 KB of LDS; k_quant_g256sf: 64)
 __global__ void k_act_w4a8(const float *x, int M, int K, int gsize, int8_t *xq, float *ascale, int *xqsum64, const float *u,
                            float *h);
-__global__ void k_act_x24(const float *x, int M, int K, int8_t *xd, float *xs, int *dsum);
+__global__ void k_act_x24(const float *x, int M, int K, int8_t *xd, float *xs, int *dsum, const float *u, float *h);
 __global__ void k_act_import_i8(const int8_t *xq, const float *ascale, int M, int K, int gq, int split, int8_t *xw,
                                 float *xs, int *xsum64);
 __global__ void k_quant_q4g64(const float *w, int N, int K, uint8_t *packed, float *scales);
@@ -215,7 +216,7 @@ __global__ void k_quant_q4g32h(const float *w, int N, int K, uint8_t *packed, ui
 __global__ void k_quant_g256sf(const float *w, int N, int K, uint8_t *packed, float *wsuper, uint8_t *sub);
 __global__ void k_repack_nib(const uint8_t *src, int N, int K, uint32_t flip, uint8_t *dst);
 __global__ void k_repack_q8(const int8_t *src, int N, int K, uint8_t *dst);
-__global__ void k_repack_qng(const uint8_t *src, int N, int K, int n, uint8_t *dst);
+void bgl_repack_qng(const uint8_t *src, int N, int K, int n, uint8_t *dst, hipStream_t st);
 __global__ void k_repack_u32(const uint32_t *src, int N, int U, uint32_t *dst);
 __global__ void k_repack_u64(const uint64_t *src, int N, int U, uint64_t *dst);
 __global__ void k_repack_zip_u32(const uint32_t *a, const uint32_t *b, int N, int U, uint2 *dst);

@@ -6,7 +6,8 @@
 //   g, u = W_gate x, W_up x      bgl_matmul_group_dev over {gate, up} (one fused launch)
 //   h = silu(g) * u              k_swiglu: h = (g / (1 + exp(-g))) * u in fp32, exp rounded once
 //                                (several W4A8 columns whose down projection quantizes them up front:
-//                                that quantization launch forms h itself, so no k_swiglu launch)
+//                                that quantization launch forms h itself, so no k_swiglu launch; fp32
+//                                columns whose down projection multiplies prepared digits: so does theirs)
 //                                (several fp32 columns on the matrix cores: the GEMM's reduce launch
 //                                forms h with the same arithmetic, from the K-split sums or, for a
 //                                tensor whose K did not split, from the g / u the GEMM stored)
@@ -81,6 +82,11 @@ extern "C" int bgl_mlp_dev(bgl_ctx *c, const bgl_tensor *gate, const bgl_tensor 
     // several W4A8 columns whose down projection quantizes them up front: that launch forms h too
     if (act == BGL_ACT_W4A8) {
         rc = run_down_swiglu_w4a8(c, down->T, g, u, h, M, y_dev);
+        if (rc <= 0) return rc;
+    }
+    // fp32 columns whose down projection multiplies prepared digits: so does theirs
+    if (act == BGL_ACT_F32) {
+        rc = run_down_swiglu_f32(c, down, g, u, h, M, y_dev);
         if (rc <= 0) return rc;
     }
     int tok = prof_begin(c, 2);

@@ -344,7 +344,7 @@ static int moe_prep(bgl_ctx *c, int slot, const float *x_dev, int M, int K, Gemv
         return bgl_last_code();
     int tok = prof_begin(c, 0);
     hipLaunchKernelGGL(k_act_x24, dim3(nblk((long)M * ng * 64)), dim3(256), 0, c->stream, x_dev, M, K, (int8_t *)w.p,
-                       (float *)s.p, (int *)d.p);
+                       (float *)s.p, (int *)d.p, (const float *)nullptr, (float *)nullptr);
     prof_end(c, tok);
     HIPCHK(hipGetLastError());
     memset(&A, 0, sizeof A);

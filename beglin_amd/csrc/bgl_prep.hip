@@ -74,6 +74,7 @@ __global__ __launch_bounds__(256) void k_act_w4a8(const float *__restrict__ x, i
 //   xd   [m][g][digit][64] bytes, then the level-1 digits;
 //   xs   [m][g] = 2^(e-22), then [m][g] = 2^(e1-22) (0 without level 1);
 //   dsum [m][K/32][4] per-half digit sums (the 4th int: the group's BGL_XF_* flags), then level 1's.
+// u != null: the column is h = silu(x) * u of the MLP block, also written to h (as k_act_w4a8).
 __device__ __forceinline__ int x_balanced3(int X, int &d0, int &d1) {
     d0 = (int)(int8_t)(X & 255);
     const int X1 = (X - d0) >> 8;
@@ -83,12 +84,18 @@ __device__ __forceinline__ int x_balanced3(int X, int &d0, int &d1) {
 
 __global__ __launch_bounds__(256) void k_act_x24(const float *__restrict__ x, int M, int K,
                                                  int8_t *__restrict__ xd, float *__restrict__ xs,
-                                                 int *__restrict__ dsum) {
+                                                 int *__restrict__ dsum, const float *__restrict__ u, float *__restrict__ h) {
     int wid = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
     int ng = K >> 6;
     if (wid >= M * ng) return;
     int m = wid / ng, g = wid % ng;
-    float v = x[(size_t)m * K + (size_t)g * 64 + lane];
+    const size_t o = (size_t)m * K + (size_t)g * 64 + lane;
+    float v = x[o];
+    if (u) {                                               // h = silu(x) * u: k_swiglu's arithmetic
+        const float e = (float)exp(-(double)v);
+        v = __fmul_rn(__fdiv_rn(v, __fadd_rn(1.0f, e)), u[o]);
+        h[o] = v;
+    }
     uint32_t ab = __float_as_uint(v) & 0x7fffffffu;
     const bool nf = ab >= 0x7f800000u;                     // NaN or +-Inf: 0 in the digits
     if (nf) { v = 0.0f; ab = 0u; }
@@ -165,67 +172,113 @@ __global__ __launch_bounds__(256) void k_act_import_i8(const int8_t *__restrict_
 }
 
 // ------------------------------------------------------------------ device packers (reference byte layouts)
-// One thread per (row, group).  Arithmetic identical to the reference packers.
+// One thread per (row, group), its arithmetic identical to the reference packers' and, with error
+// feedback, a chain over the group's values.  The groups of a workgroup are one run of memory (K is a
+// whole number of groups), so they are read coalesced into LDS first, one word of padding per group (a
+// thread walking its own group in memory touches a line per lane and value: k_quant_q4g64 over 14336 x
+// 4096 took 185 us, 71 us staged; a plain read of the 235 MB takes 46).
+typedef float pk_f4 __attribute__((ext_vector_type(4), aligned(4)));   // the caller's rows: a float's alignment
+template <int G, int NT>
+__device__ __forceinline__ const float *stage_groups(const float *__restrict__ w, long t0, long total, float *lds) {
+    constexpr int IT = G / 4, BT = IT < 16 ? IT : 16;             // 16-byte loads per thread, a batch in flight
+#pragma unroll
+    for (int i0 = 0; i0 < IT; i0 += BT) {
+        pk_f4 v[BT];
+#pragma unroll
+        for (int j = 0; j < BT; j++) {
+            const int i = threadIdx.x + (i0 + j) * NT, g = i / IT, p = 4 * (i % IT);
+            v[j] = *reinterpret_cast<const pk_f4 *>(w + (t0 + g < total ? t0 + g : total - 1) * G + p);
+        }
+#pragma unroll
+        for (int j = 0; j < BT; j++) {
+            const int i = threadIdx.x + (i0 + j) * NT, g = i / IT, p = 4 * (i % IT);
+            float *d = lds + g * (G + 1) + p;
+            d[0] = v[j].x; d[1] = v[j].y; d[2] = v[j].z; d[3] = v[j].w;
+        }
+    }
+    __syncthreads();
+    return lds + threadIdx.x * (G + 1);
+}
+// C values with error feedback into C / 8 dwords of nibbles (code + 8; even value low)
+template <int C>
+__device__ __forceinline__ void pack_nibbles(const float *grp, float scale, float inv, float &err, uint32_t *b) {
+#pragma unroll
+    for (int j = 0; j < C / 8; j++) {
+        uint32_t v = 0;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            float xv = __fadd_rn(grp[8 * j + i], err);
+            float qf = rintf(__fmul_rn(xv, inv));
+            qf = fminf(fmaxf(qf, -8.0f), 7.0f);
+            err = __fsub_rn(xv, __fmul_rn(qf, scale));
+            v |= (uint32_t)(((int)qf + 8) & 15) << (4 * i);
+        }
+        b[j] = v;
+    }
+}
 
 // gguf_transcode.c:24-68 (q4g64 with error feedback).
-__global__ void k_quant_q4g64(const float *__restrict__ w, int N, int K, uint8_t *__restrict__ packed,
+__global__ __launch_bounds__(PK_THREADS) void k_quant_q4g64(const float *__restrict__ w, int N, int K, uint8_t *__restrict__ packed,
                               float *__restrict__ scales) {
-    int ng = K / 64;
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long)N * ng) return;
-    int r = (int)(t / ng), g = (int)(t % ng);
-    const float *grp = w + (size_t)r * K + (size_t)g * 64;
+    __shared__ float lds[PK_THREADS * 65];
+    const long total = (long)N * (K / 64), t0 = (long)blockIdx.x * blockDim.x, t = t0 + threadIdx.x;
+    const float *grp = stage_groups<64, PK_THREADS>(w, t0, total, lds);
+    if (t >= total) return;
     float maxabs = 0.0f;
+#pragma unroll 16
     for (int p = 0; p < 64; p++) maxabs = fmaxf(maxabs, fabsf(grp[p]));
     float scale = __fdiv_rn(maxabs, 7.0f);
     if (scale < 1e-12f) scale = 1.0f;
     scales[t] = scale;
     float inv = __fdiv_rn(1.0f, scale), err = 0.0f;
-    uint8_t *prow = packed + (size_t)r * (K / 2) + (size_t)g * 32;
-    for (int p = 0; p < 64; p += 2) {
-        int nib[2];
-        for (int h = 0; h < 2; h++) {
-            float xv = __fadd_rn(grp[p + h], err);
-            float qf = rintf(__fmul_rn(xv, inv));
-            qf = fminf(fmaxf(qf, -8.0f), 7.0f);
-            err = __fsub_rn(xv, __fmul_rn(qf, scale));
-            nib[h] = ((int)qf + 8) & 15;
-        }
-        prow[p / 2] = (uint8_t)(nib[0] | (nib[1] << 4));
+    uint4 *dst = reinterpret_cast<uint4 *>(packed + (size_t)t * 32);
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        uint32_t b[4];
+        pack_nibbles<32>(grp + 32 * k, scale, inv, err, b);
+        dst[k] = make_uint4(b[0], b[1], b[2], b[3]);
     }
 }
 
 // gguf_transcode.c:70-101 (q8g64: direct division, no error feedback).
-__global__ void k_quant_q8g64(const float *__restrict__ w, int N, int K, int8_t *__restrict__ codes,
+__global__ __launch_bounds__(PK_THREADS) void k_quant_q8g64(const float *__restrict__ w, int N, int K, int8_t *__restrict__ codes,
                               float *__restrict__ scales) {
-    int ng = K / 64;
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long)N * ng) return;
-    int r = (int)(t / ng), g = (int)(t % ng);
-    const float *grp = w + (size_t)r * K + (size_t)g * 64;
+    __shared__ float lds[PK_THREADS * 65];
+    const long total = (long)N * (K / 64), t0 = (long)blockIdx.x * blockDim.x, t = t0 + threadIdx.x;
+    const float *grp = stage_groups<64, PK_THREADS>(w, t0, total, lds);
+    if (t >= total) return;
     float maxabs = 0.0f;
+#pragma unroll 16
     for (int p = 0; p < 64; p++) maxabs = fmaxf(maxabs, fabsf(grp[p]));
     float scale = __fdiv_rn(maxabs, 127.0f);
     if (scale < 1e-12f) scale = 1.0f;
     scales[t] = scale;
-    int8_t *c = codes + (size_t)r * K + (size_t)g * 64;
-    for (int p = 0; p < 64; p++) {
-        float qf = rintf(__fdiv_rn(grp[p], scale));
-        qf = fminf(fmaxf(qf, -127.0f), 127.0f);
-        c[p] = (int8_t)qf;
+    uint4 *dst = reinterpret_cast<uint4 *>(codes + (size_t)t * 64);
+    for (int k = 0; k < 4; k++) {
+        uint32_t b[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            b[j] = 0;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                float qf = rintf(__fdiv_rn(grp[16 * k + 4 * j + i], scale));
+                qf = fminf(fmaxf(qf, -127.0f), 127.0f);
+                b[j] |= (uint32_t)(uint8_t)(int8_t)qf << (8 * i);
+            }
+        }
+        dst[k] = make_uint4(b[0], b[1], b[2], b[3]);
     }
 }
 
 // gguf_transcode.c:108-162 (dense_floor=0) or qng64_dense.c:29-68 (dense_floor=1): the two
 // qNg64 encoders differ only in the scale floor test.
-__global__ void k_quant_qng64(const float *__restrict__ w, int N, int K, int n, int dense_floor,
+__global__ __launch_bounds__(PK_THREADS) void k_quant_qng64(const float *__restrict__ w, int N, int K, int n, int dense_floor,
                               uint8_t *__restrict__ planes, float *__restrict__ scales) {
-    int ng = K / 64;
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long)N * ng) return;
-    int r = (int)(t / ng), g = (int)(t % ng);
+    __shared__ float lds[PK_THREADS * 65];
+    const long total = (long)N * (K / 64), t0 = (long)blockIdx.x * blockDim.x, t = t0 + threadIdx.x;
+    const float *grp = stage_groups<64, PK_THREADS>(w, t0, total, lds);
+    if (t >= total) return;
     int qmax = (1 << (n - 1)) - 1, qmin = -(1 << (n - 1)), bias = 1 << (n - 1), mask = (1 << n) - 1;
-    const float *grp = w + (size_t)r * K + (size_t)g * 64;
     float maxabs = 0.0f;
     for (int p = 0; p < 64; p++) maxabs = fmaxf(maxabs, fabsf(grp[p]));
     float scale;
@@ -233,87 +286,76 @@ __global__ void k_quant_qng64(const float *__restrict__ w, int N, int K, int n, 
     else { scale = __fdiv_rn(maxabs, (float)qmax); if (scale < 1e-12f) scale = 1.0f; }
     scales[t] = scale;
     float inv = __fdiv_rn(1.0f, scale), err = 0.0f;
-    uint32_t pl[15][2];
-    for (int j = 0; j < 15; j++) { pl[j][0] = 0; pl[j][1] = 0; }
-    for (int p = 0; p < 64; p++) {
-        float xv = __fadd_rn(grp[p], err);
-        float qf = rintf(__fmul_rn(xv, inv));
-        qf = fminf(fmaxf(qf, (float)qmin), (float)qmax);
-        err = __fsub_rn(xv, __fmul_rn(qf, scale));
-        uint32_t u = (uint32_t)(((int)qf + bias) & mask);
-        for (int j = 0; j < n; j++) pl[j][p >> 5] |= ((u >> j) & 1u) << (p & 31);
+    uint32_t *dst = reinterpret_cast<uint32_t *>(planes + (size_t)t * (size_t)n * 8);
+    for (int h = 0; h < 2; h++) {                          // values 0..31, 32..63: dword h of every plane
+        uint32_t pl[15];
+#pragma unroll
+        for (int j = 0; j < 15; j++) pl[j] = 0;
+        for (int p = 0; p < 32; p++) {
+            float xv = __fadd_rn(grp[32 * h + p], err);
+            float qf = rintf(__fmul_rn(xv, inv));
+            qf = fminf(fmaxf(qf, (float)qmin), (float)qmax);
+            err = __fsub_rn(xv, __fmul_rn(qf, scale));
+            uint32_t u = (uint32_t)(((int)qf + bias) & mask);
+#pragma unroll
+            for (int j = 0; j < 15; j++) pl[j] |= ((u >> j) & 1u) << p;
+        }
+#pragma unroll
+        for (int j = 0; j < 15; j++)
+            if (j < n) dst[2 * j + h] = pl[j];
     }
-    uint32_t *dst = reinterpret_cast<uint32_t *>(planes + ((size_t)r * ng + g) * (size_t)n * 8);
-    for (int j = 0; j < n; j++) { dst[2 * j] = pl[j][0]; dst[2 * j + 1] = pl[j][1]; }
 }
 
 // gguf_write_quants.c:34-62 (Q4_0 encoder: fp32 scale inside the loop, fp16 stored), written in
 // the Q4G32H pairing (byte b low = element 2b, high = 2b+1) with the fp16 scale beside it.
-__global__ void k_quant_q4g32h(const float *__restrict__ w, int N, int K, uint8_t *__restrict__ packed,
+__global__ __launch_bounds__(PK_THREADS) void k_quant_q4g32h(const float *__restrict__ w, int N, int K, uint8_t *__restrict__ packed,
                                uint16_t *__restrict__ scales16) {
-    int nb = K / 32;
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long)N * nb) return;
-    int r = (int)(t / nb), b = (int)(t % nb);
-    const float *grp = w + (size_t)r * K + (size_t)b * 32;
+    __shared__ float lds[PK_THREADS * 33];
+    const long total = (long)N * (K / 32), t0 = (long)blockIdx.x * blockDim.x, t = t0 + threadIdx.x;
+    const float *grp = stage_groups<32, PK_THREADS>(w, t0, total, lds);
+    if (t >= total) return;
     float maxabs = 0.0f;
+#pragma unroll 16
     for (int p = 0; p < 32; p++) maxabs = fmaxf(maxabs, fabsf(grp[p]));
     float scale = __fdiv_rn(maxabs, 7.0f);
     if (scale < 1e-12f) scale = 1.0f;
     scales16[t] = __half_as_ushort(__float2half_rn(scale));
     float inv = __fdiv_rn(1.0f, scale), err = 0.0f;
-    uint8_t *dst = packed + (size_t)r * (K / 2) + (size_t)b * 16;
-    for (int p = 0; p < 32; p += 2) {
-        int nib[2];
-        for (int h = 0; h < 2; h++) {
-            float xv = __fadd_rn(grp[p + h], err);
-            float qf = rintf(__fmul_rn(xv, inv));
-            qf = fminf(fmaxf(qf, -8.0f), 7.0f);
-            err = __fsub_rn(xv, __fmul_rn(qf, scale));
-            nib[h] = ((int)qf + 8) & 15;
-        }
-        dst[p / 2] = (uint8_t)(nib[0] | (nib[1] << 4));
-    }
+    uint32_t b[4];
+    pack_nibbles<32>(grp, scale, inv, err, b);
+    *reinterpret_cast<uint4 *>(packed + (size_t)t * 16) = make_uint4(b[0], b[1], b[2], b[3]);
 }
 
 // q4g256sf (build-defined packer; same arithmetic as the oracle's or_quantize_g256sf): one thread
 // per (row, superblock).
-__global__ void k_quant_g256sf(const float *__restrict__ w, int N, int K, uint8_t *__restrict__ packed,
+__global__ __launch_bounds__(64) void k_quant_g256sf(const float *__restrict__ w, int N, int K, uint8_t *__restrict__ packed,
                                float *__restrict__ wsuper, uint8_t *__restrict__ sub) {
-    int ns = K / 256;
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long)N * ns) return;
-    int r = (int)(t / ns), gs = (int)(t % ns);
-    const float *row = w + (size_t)r * K;
+    __shared__ float lds[64 * 257];
+    const long total = (long)N * (K / 256), t0 = (long)blockIdx.x * blockDim.x, t = t0 + threadIdx.x;
+    const float *row = stage_groups<256, 64>(w, t0, total, lds);
+    if (t >= total) return;
     float s64[4], ws = 0.0f;
     for (int k = 0; k < 4; k++) {
-        const float *grp = row + (size_t)(gs * 4 + k) * 64;
         float maxabs = 0.0f;
-        for (int p = 0; p < 64; p++) maxabs = fmaxf(maxabs, fabsf(grp[p]));
+#pragma unroll 16
+        for (int p = 0; p < 64; p++) maxabs = fmaxf(maxabs, fabsf(row[64 * k + p]));
         s64[k] = __fdiv_rn(maxabs, 7.0f);
         ws = fmaxf(ws, s64[k]);
     }
     if (ws < 1e-12f) ws = 1.0f;
     wsuper[t] = ws;
     for (int k = 0; k < 4; k++) {
-        int g = gs * 4 + k;
         int sc = (int)ceilf(__fdiv_rn(__fmul_rn(63.0f, s64[k]), ws));
         sc = sc < 1 ? 1 : (sc > 63 ? 63 : sc);
-        sub[(size_t)r * (K / 64) + g] = (uint8_t)sc;
+        sub[(size_t)t * 4 + k] = (uint8_t)sc;
         float scale = __fmul_rn(ws, __fdiv_rn((float)sc, 63.0f));
         float inv = __fdiv_rn(1.0f, scale), err = 0.0f;
-        const float *grp = row + (size_t)g * 64;
-        uint8_t *dst = packed + (size_t)r * (K / 2) + (size_t)g * 32;
-        for (int p = 0; p < 64; p += 2) {
-            int nib[2];
-            for (int h = 0; h < 2; h++) {
-                float xv = __fadd_rn(grp[p + h], err);
-                float qf = rintf(__fmul_rn(xv, inv));
-                qf = fminf(fmaxf(qf, -8.0f), 7.0f);
-                err = __fsub_rn(xv, __fmul_rn(qf, scale));
-                nib[h] = ((int)qf + 8) & 15;
-            }
-            dst[p / 2] = (uint8_t)(nib[0] | (nib[1] << 4));
+        uint4 *dst = reinterpret_cast<uint4 *>(packed + (size_t)t * 128 + 32 * k);
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            uint32_t b[4];
+            pack_nibbles<32>(row + 64 * k + 32 * j, scale, inv, err, b);
+            dst[j] = make_uint4(b[0], b[1], b[2], b[3]);
         }
     }
 }
@@ -365,73 +407,79 @@ __global__ void k_repack_q8(const int8_t *__restrict__ src, int N, int K, uint8_
 // order), the 2-bit field (2 chunks; dword j byte i crumb t = element 16j+4t+i of the 64-group) and
 // the 1-bit field (1 chunk; dword j byte i bit t = element 32j+4t+i of the pair).  A missing second
 // group (odd K/64) is padded with u = 0.
-__global__ void k_repack_qng(const uint8_t *__restrict__ src, int N, int K, int n, uint8_t *__restrict__ dst) {
-    int ng = K / 64, np = (ng + 1) / 2;
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    long ntiles = (N + BGL_TILE - 1) / BGL_TILE;
-    if (t >= ntiles * BGL_TILE * np) return;
-    int r = (int)(t / np), pr = (int)(t % np);
-    QngFields f = qng_fields(n);
-    uint16_t u[128];
-    for (int e = 0; e < 128; e++) u[e] = 0;
-    if (r < N)
-        for (int h = 0; h < 2; h++) {
-            int g = 2 * pr + h;
-            if (g >= ng) break;
-            const uint8_t *grp = src + ((size_t)r * ng + g) * (size_t)n * 8;
-            for (int p = 0; p < 64; p++) {
-                uint32_t v = 0;
-                for (int j = 0; j < n; j++) v |= (uint32_t)((grp[j * 8 + (p >> 3)] >> (p & 7)) & 1) << j;
-                u[64 * h + p] = (uint16_t)v;
-            }
-        }
-    int tile = r / BGL_TILE, lane = r % BGL_TILE;
-    int cpr = np * n, c = pr * n;
-    auto put = [&](int chunk, const uint32_t *wv) {
-        uint4 *d = reinterpret_cast<uint4 *>(dst + (((size_t)tile * cpr + chunk) * BGL_TILE + lane) * 16);
-        *d = make_uint4(wv[0], wv[1], wv[2], wv[3]);
+// One thread per (64-row tile, group, row), rows along the lanes so every store is one 1 KB run.  Four
+// consecutive values sit in the four bytes of one dword in every field, so plane j's bits 4m..4m+3 are
+// spread into bytes (x * 0x204081 puts bit i at 8i) and shifted into their field.  (Value by value
+// through a local array: 4139 us for 14336 x 4096 at n = 7, 22 us so.)
+template <int NB>
+__global__ __launch_bounds__(256) void k_repack_qng(const uint8_t *__restrict__ src, int N, int K, uint8_t *__restrict__ dst) {
+    constexpr int H8 = (NB >> 3) & 1, H4 = (NB >> 2) & 1, H2 = (NB >> 1) & 1, H1 = NB & 1;
+    const int ng = K / 64, np = (ng + 1) / 2;
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long ntiles = (N + BGL_TILE - 1) / BGL_TILE;
+    if (t >= ntiles * BGL_TILE * np * 2) return;
+    const int lane = (int)(t % BGL_TILE), g = (int)((t / BGL_TILE) % (2 * np)), tile = (int)(t / BGL_TILE / (2 * np));
+    const int r = tile * BGL_TILE + lane, h = g & 1;
+    uint32_t pl[NB][2];
+#pragma unroll
+    for (int j = 0; j < NB; j++) { pl[j][0] = 0; pl[j][1] = 0; }
+    if (r < N && g < ng) {
+        const uint2 *grp = reinterpret_cast<const uint2 *>(src + ((size_t)r * ng + g) * (size_t)NB * 8);
+#pragma unroll
+        for (int j = 0; j < NB; j++) { const uint2 v = grp[j]; pl[j][0] = v.x; pl[j][1] = v.y; }
+    }
+    uint8_t *base = dst + ((size_t)tile * np * NB + (size_t)(g >> 1) * NB) * 1024 + lane * 16;
+    // planes [j0, j0 + W) of values 4m..4m+3 as a W-bit number per byte
+    auto field = [&](int j0, int W, int m) {
+        uint32_t v = 0;
+#pragma unroll
+        for (int j = 0; j < W; j++) v |= ((((pl[j0 + j][m >> 3] >> (4 * (m & 7))) & 15u) * 0x204081u) & 0x01010101u) << j;
+        return v;
     };
-    uint32_t wv[4];
-    if (f.has8)
-        for (int k = 0; k < 8; k++, c++) {
-            for (int j = 0; j < 4; j++) {
-                wv[j] = 0;
-                for (int i = 0; i < 4; i++) wv[j] |= (uint32_t)(((u[16 * k + 4 * j + i]) & 255) ^ 0x80) << (8 * i);
-            }
-            put(c, wv);
+    auto put = [&](int chunk, const uint32_t (&w)[4]) { *reinterpret_cast<uint4 *>(base + (size_t)chunk * 1024) = make_uint4(w[0], w[1], w[2], w[3]); };
+    uint32_t w[4];
+    if constexpr (H8)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {                      // 16 values per chunk
+#pragma unroll
+            for (int j = 0; j < 4; j++) w[j] = field(0, 8, 4 * k + j) ^ 0x80808080u;
+            put(4 * h + k, w);
         }
-    if (f.has4)
-        for (int k = 0; k < 4; k++, c++) {
-            for (int j = 0; j < 4; j++) {
-                wv[j] = 0;
-                for (int i = 0; i < 4; i++) {
-                    uint32_t lo = (u[32 * k + 8 * j + i] >> f.sh4) & 15, hi = (u[32 * k + 8 * j + 4 + i] >> f.sh4) & 15;
-                    wv[j] |= (lo | (hi << 4)) << (8 * i);
-                }
-            }
-            put(c, wv);
+    if constexpr (H4)
+#pragma unroll
+        for (int k = 0; k < 2; k++) {                      // 32 values: low nibbles 8j..8j+3, high 8j+4..8j+7
+#pragma unroll
+            for (int j = 0; j < 4; j++) w[j] = field(8 * H8, 4, 8 * k + 2 * j) | (field(8 * H8, 4, 8 * k + 2 * j + 1) << 4);
+            put(8 * H8 + 2 * h + k, w);
         }
-    if (f.has2)
-        for (int k = 0; k < 2; k++, c++) {
-            for (int j = 0; j < 4; j++) {
-                wv[j] = 0;
-                for (int i = 0; i < 4; i++)
-                    for (int q = 0; q < 4; q++)
-                        wv[j] |= (uint32_t)((u[64 * k + 16 * j + 4 * q + i] >> f.sh2) & 3) << (8 * i + 2 * q);
-            }
-            put(c, wv);
-        }
-    if (f.has1) {
+    if constexpr (H2) {                                    // 64 values: crumb q of dword j = 16j + 4q ..
+#pragma unroll
         for (int j = 0; j < 4; j++) {
-            wv[j] = 0;
-            for (int i = 0; i < 4; i++)
-                for (int q = 0; q < 8; q++)
-                    wv[j] |= (uint32_t)((u[32 * j + 4 * q + i] >> f.sh1) & 1) << (8 * i + q);
+            w[j] = 0;
+#pragma unroll
+            for (int q = 0; q < 4; q++) w[j] |= field(8 * H8 + 4 * H4, 2, 4 * j + q) << (2 * q);
         }
-        put(c, wv);
-        c++;
+        put(8 * H8 + 4 * H4 + h, w);
+    }
+    if constexpr (H1) {                                    // both groups' 64 values in one chunk: bit q of dword j = 32j + 4q ..
+        uint32_t b[2] = {0, 0};
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int q = 0; q < 8; q++) b[j] |= field(8 * H8 + 4 * H4 + 2 * H2, 1, 8 * j + q) << q;
+        *reinterpret_cast<uint2 *>(base + (size_t)(8 * H8 + 4 * H4 + 2 * H2) * 1024 + 8 * h) = make_uint2(b[0], b[1]);
     }
 }
+
+template <int NB>
+static void repack_qng_launch(const uint8_t *src, int N, int K, int n, uint8_t *dst, hipStream_t st) {
+    if constexpr (NB <= 15) {
+        if (n != NB) return repack_qng_launch<NB + 1>(src, N, K, n, dst, st);
+        const long ntiles = (N + BGL_TILE - 1) / BGL_TILE, threads = ntiles * BGL_TILE * ((K / 64 + 1) / 2) * 2;
+        hipLaunchKernelGGL((k_repack_qng<NB>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, src, N, K, dst);
+    }
+}
+void bgl_repack_qng(const uint8_t *src, int N, int K, int n, uint8_t *dst, hipStream_t st) { repack_qng_launch<2>(src, N, K, n, dst, st); }
 
 // Per-(row, unit) scalars [N][U] (32-bit words) -> [tile][U][lane]; padded rows get 0.
 __global__ void k_repack_u32(const uint32_t *__restrict__ src, int N, int U, uint32_t *__restrict__ dst) {
@@ -505,11 +553,61 @@ __global__ void k_repack_qng_scales(const float *__restrict__ src, int N, int ng
 }
 
 // ------------------------------------------------------------------ dequant probe (tiled layout)
-// Decodes rows [row0, row0+nrows) of a bound tensor straight from the device layout, one thread
-// per element -- the device analogue of moe_decode_af (qwen_infer.c:2554-2655) used to prove that
+// Decodes rows [row0, row0+nrows) of a bound tensor straight from the device layout -- the device analogue of moe_decode_af (qwen_infer.c:2554-2655) used to prove that
 // the repacked layout decodes bit-exactly.
-__global__ void k_dequant(BglDevTensor T, int row0, int nrows, float *__restrict__ out) {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long)nrows * T.K) return;
-    out[t] = w_at(T, row0 + (int)(t / T.K), (int)(t % T.K));
+// A workgroup decodes 16 rows x 64 columns, a thread 4 consecutive columns (one value per thread, with a
+// 64-bit division to find it, took 150 us for 14336 x 4096 q4g64; 40 us so, 46 for a plain write).
+// int4: the 4 columns are the low or the high nibbles of one dword.
+__global__ __launch_bounds__(256) void k_dequant(BglDevTensor T, int row0, int nrows, float *__restrict__ out) {
+    const unsigned ng = T.K / 64;                            // workgroups along the columns
+    const int rl = (int)(blockIdx.x / ng) * 16 + (threadIdx.x >> 4), c = (int)(blockIdx.x % ng) * 64 + 4 * (threadIdx.x & 15);
+    if (rl >= nrows) return;
+    const int r = row0 + rl, tile = r / BGL_TILE, lane = r % BGL_TILE;
+    pk_f4 v;
+    if (T.fmt == BGL_Q4G64 || T.fmt == BGL_Q4G32H || T.fmt == BGL_Q4G256SF) {
+        const uint32_t d = *reinterpret_cast<const uint32_t *>(T.w + (((size_t)tile * T.cpr + c / 32) * BGL_TILE + lane) * 16 + 4 * ((c % 32) / 8));
+        uint32_t n4 = c % 8 ? (d >> 4) & 0x0F0F0F0Fu : d & 0x0F0F0F0Fu;
+        if (T.fmt == BGL_Q4G256SF) n4 ^= 0x08080808u;        // stored as signed nibbles
+        float s;
+        if (T.fmt == BGL_Q4G64) {
+            s = reinterpret_cast<const float *>(T.s0)[((size_t)tile * T.nunits + c / 64) * BGL_TILE + lane];
+        } else if (T.fmt == BGL_Q4G32H) {
+            const uint32_t s2 = reinterpret_cast<const uint32_t *>(T.s0)[((size_t)tile * T.nunits + c / 64) * BGL_TILE + lane];
+            s = __half2float(__ushort_as_half((unsigned short)((c / 32) & 1 ? s2 >> 16 : s2 & 0xffff)));
+        } else {
+            const uint2 ws = reinterpret_cast<const uint2 *>(T.s0)[((size_t)tile * T.nunits + c / 256) * BGL_TILE + lane];
+            const float sc = (float)((ws.y >> (8 * ((c / 64) & 3))) & 255);
+            s = T.gmul == 1.0f ? __uint_as_float(ws.x) : __fmul_rn(__uint_as_float(ws.x), __fdiv_rn(sc, 63.0f));
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = __fmul_rn((float)((int)((n4 >> (8 * i)) & 15) - 8), s);
+    } else if (T.fmt == BGL_Q8G64) {
+        const uint32_t d = *reinterpret_cast<const uint32_t *>(T.w + (((size_t)tile * T.cpr + c / 16) * BGL_TILE + lane) * 16 + c % 16);
+        const float s = reinterpret_cast<const float *>(T.s0)[((size_t)tile * T.nunits + c / 64) * BGL_TILE + lane];
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = __fmul_rn((float)(int8_t)(d >> (8 * i)), s);
+    } else if (T.fmt == BGL_QNG64) {                         // in every field the 4 columns are the bytes of one dword
+        const QngFields f = qng_fields(T.bits);
+        const int e = c % 128;
+        const uint8_t *p = T.w + (((size_t)tile * T.cpr + (size_t)(c / 128) * T.bits) * BGL_TILE + lane) * 16;
+        auto dw = [&](int chunk, int j) { return *reinterpret_cast<const uint32_t *>(p + (size_t)chunk * 1024 + 4 * j); };
+        uint32_t b8 = 0, b4 = 0, b2 = 0, b1 = 0;
+        int k = 0;
+        if (f.has8) { b8 = dw(k + e / 16, (e % 16) / 4) ^ 0x80808080u; k += 8; }
+        if (f.has4) { b4 = (dw(k + e / 32, (e % 32) / 8) >> (e % 8 ? 4 : 0)) & 0x0F0F0F0Fu; k += 4; }
+        if (f.has2) { b2 = (dw(k + e / 64, (e % 64) / 16) >> (2 * ((e % 16) / 4))) & 0x03030303u; k += 2; }
+        if (f.has1) b1 = (dw(k, e / 32) >> ((e % 32) / 4)) & 0x01010101u;
+        const float2 s2 = reinterpret_cast<const float2 *>(T.s0)[((size_t)tile * T.nunits + c / 128) * BGL_TILE + lane];
+        const float s = e / 64 ? s2.y : s2.x;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t u = ((b8 >> (8 * i)) & 255) | (((b4 >> (8 * i)) & 255) << f.sh4) | (((b2 >> (8 * i)) & 255) << f.sh2) |
+                               (((b1 >> (8 * i)) & 255) << f.sh1);
+            v[i] = __fmul_rn((float)((int)u - (1 << (T.bits - 1))), s);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = w_at(T, r, c + i);
+    }
+    *reinterpret_cast<pk_f4 *>(out + (size_t)rl * T.K + c) = v;
 }
