@@ -45,8 +45,8 @@
 
 #include <algorithm>
 
-#include "bgl_gemv_impl.h"
 #include "bgl_internal.h"
+#include "bgl_mfma_a.h"
 
 #define HIPCHK(expr)                                                                             \
     do {                                                                                         \
@@ -54,19 +54,11 @@
         if (e_ != hipSuccess) return bgl_fail(BGL_E_HIP, "%s: %s", #expr, hipGetErrorString(e_)); \
     } while (0)
 
-typedef _Float16 mf_h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 mf_h2 __attribute__((ext_vector_type(2)));
-typedef float mf_f4 __attribute__((ext_vector_type(4)));
-typedef unsigned int mf_u4 __attribute__((ext_vector_type(4)));
-typedef unsigned int mf_u2 __attribute__((ext_vector_type(2)));
-
 #define MF_TILES 4           // 64-row weight tiles per workgroup (they share the staged activations)
-#define MF_RBW 2             // 16-row blocks per wave: two waves per tile
 #define MF_WAVES (MF_TILES * 4 / MF_RBW)
 #define MF_KSTEP_PAD 16      // split length granularity in K-steps (every ring depth divides it)
 #define MF_MAXCT 4           // column tiles (16 columns each) per launch: up to 64 columns
 #define MF_MAXN 10           // qNg64 widths whose codes are exact in fp16 via the 1024+u trick
-#define MF_RSRC_W3 0x00020000   // buffer resource word 3 on gfx9: 32-bit data format, raw addressing
 
 struct MfmaTask {
     BglDevTensor T;
@@ -86,213 +78,6 @@ struct MfmaLaunch {
     const float *x;          // activations x[m][k], M rows of K floats
 };
 
-// ==================================================================================== weights
-// Raw A-fragment words of one K-step for one lane (row 16*rb + lane%16, slot q = lane/16).
-template <int FMT, int NB> struct ARaw { uint32_t w[1]; };
-template <int NB> struct ARaw<BGL_Q8G64, NB> { uint32_t w[2]; };
-template <int NB> struct ARaw<BGL_QNG64, NB> {
-    static constexpr int H8 = (NB >> 3) & 1, H4 = (NB >> 2) & 1, H2 = (NB >> 1) & 1, H1 = NB & 1;
-    uint32_t w[2 * H8 + H4 + H2 + H1 > 0 ? 2 * H8 + H4 + H2 + H1 : 1];
-};
-
-template <int FMT> constexpr int ksteps_per_unit() { return FMT == BGL_QNG64 ? 4 : 2; }
-// quantization groups per unit: two for the fp16-pair (Q4G32H) and float2 (qNg64) scale words
-template <int FMT> constexpr int groups_per_unit() { return FMT == BGL_Q4G32H || FMT == BGL_QNG64 ? 2 : 1; }
-// bytes of scale data per row and unit in the device layout
-template <int FMT> constexpr int scale_bytes() { return FMT == BGL_QNG64 ? 8 : 4; }
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t mf_rsrc(const void *p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, MF_RSRC_W3);
-}
-
-// Code planes of a format: byte codes (q8g64; qNg64 with n >= 8), nibbles (int4; qNg64 bit 2 of
-// n), crumbs and single bits (qNg64).
-template <int FMT, int NB> struct Planes {
-    static constexpr int P8 = FMT == BGL_Q8G64 ? 1 : FMT == BGL_QNG64 ? (NB >> 3) & 1 : 0;
-    static constexpr int P4 = FMT == BGL_Q4G64 || FMT == BGL_Q4G32H ? 1 : FMT == BGL_QNG64 ? (NB >> 2) & 1 : 0;
-    static constexpr int P2 = FMT == BGL_QNG64 ? (NB >> 1) & 1 : 0;
-    static constexpr int P1 = FMT == BGL_QNG64 ? NB & 1 : 0;
-    static constexpr int WORDS = 8 * P8 + 4 * P4 + 4 * P2 + 4 * P1;   // per lane and K-step pair
-};
-
-// Raw words of one K-step pair (s, s+1) for a wave's two 16-row blocks, as loaded.
-//  - byte codes and nibbles are read a whole 16-byte chunk row per lane (one buffer_load_dwordx4
-//    covers 32 rows of two chunks: lanes 32..63 take the second), so each quarter-wave reads 256
-//    contiguous bytes; the MFMA operand layout (4 lanes per row) is rebuilt with lane swaps;
-//  - crumbs and bits (2/n and 1/n of a qNg64 tensor's bytes) are read as the operand's own dword.
-template <int FMT, int NB> struct PRaw {
-    using P = Planes<FMT, NB>;
-    uint32_t w8[P::P8 ? 8 : 1];      // byte codes: K-step j of the pair in words 4j..4j+3
-    uint32_t w4[P::P4 ? 4 : 1];      // nibbles: lanes < 32 K-step s, lanes >= 32 K-step s+1
-    uint32_t w2[P::P2 ? 4 : 1];      // crumb operand word of [j][rb]
-    uint32_t w1[P::P1 ? 4 : 1];      // bit operand word of [j][rb]
-};
-
-// Per-lane byte offsets within a tile's chunk, fixed for the kernel: the chunk-row reads (rows
-// 16*rb0 + lane%32 of chunk lane/32) and the operand-dword reads of row block rb0 (rb0+1 adds
-// 256 bytes).
-struct AOff { uint32_t op, o2, o1; };
-
-__device__ __forceinline__ AOff a_offsets(int rb0, int lane) {
-    AOff o;
-    o.op = (uint32_t)(lane >> 5) * 1024u + (uint32_t)(16 * rb0 + (lane & 31)) * 16u;
-    const uint32_t row = 16 * rb0 + (lane & 15), q = lane >> 4;
-    o.o2 = row * 16 + 4 * (q >> 1);                      // crumb chunk: dword 2(j%2) + q/2
-    o.o1 = row * 16;                                     // bit chunk: dword j
-    return o;
-}
-
-// Loads K-steps s, s+1 (s even, already clamped into the tensor) of the wave's rows; tchunk is the
-// first chunk of the wave's tile.
-template <int FMT, int NB>
-__device__ __forceinline__ void ld_pair(PRaw<FMT, NB> &p, __amdgpu_buffer_rsrc_t rs, const AOff &o, uint32_t tchunk, int s) {
-    using P = Planes<FMT, NB>;
-    // both are wave-uniform; said so explicitly, so every offset below is a scalar operand (a value
-    // the compiler cannot prove uniform would wrap each load in a loop over the lanes' values)
-    tchunk = __builtin_amdgcn_readfirstlane(tchunk);
-    s = __builtin_amdgcn_readfirstlane(s);
-    if constexpr (FMT == BGL_Q8G64) {                    // K-step s is chunks 2s, 2s+1
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const mf_u4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, o.op, (tchunk + 2u * (s + j)) * 1024u, 0);
-            p.w8[4 * j] = v[0]; p.w8[4 * j + 1] = v[1]; p.w8[4 * j + 2] = v[2]; p.w8[4 * j + 3] = v[3];
-        }
-    } else if constexpr (FMT == BGL_QNG64) {
-        constexpr int K4 = 8 * P::P8, K2 = K4 + 4 * P::P4, K1 = K2 + 2 * P::P2;
-        const uint32_t u = (uint32_t)s >> 2, j0 = (uint32_t)s & 3, c0 = tchunk + u * NB;
-        if constexpr (P::P8) {
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const mf_u4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, o.op, (c0 + 2 * (j0 + j)) * 1024u, 0);
-                p.w8[4 * j] = v[0]; p.w8[4 * j + 1] = v[1]; p.w8[4 * j + 2] = v[2]; p.w8[4 * j + 3] = v[3];
-            }
-        }
-        if constexpr (P::P4) {
-            const mf_u4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, o.op, (c0 + K4 + j0) * 1024u, 0);
-            p.w4[0] = v[0]; p.w4[1] = v[1]; p.w4[2] = v[2]; p.w4[3] = v[3];
-        }
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int r = 0; r < 2; r++) {
-                const uint32_t jj = j0 + j;
-                if constexpr (P::P2)
-                    p.w2[2 * j + r] = __builtin_amdgcn_raw_buffer_load_b32(rs, o.o2 + 256u * r, (c0 + K2 + (jj >> 1)) * 1024u + 8 * (jj & 1), 0);
-                if constexpr (P::P1)
-                    p.w1[2 * j + r] = __builtin_amdgcn_raw_buffer_load_b32(rs, o.o1 + 256u * r, (c0 + K1) * 1024u + 4 * jj, 0);
-            }
-    } else {                                             // int4: K-step s is chunk s
-        const mf_u4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, o.op, (tchunk + (uint32_t)s) * 1024u, 0);
-        p.w4[0] = v[0]; p.w4[1] = v[1]; p.w4[2] = v[2]; p.w4[3] = v[3];
-    }
-}
-
-// Operand words of both K-steps and row blocks from a loaded pair.  Nibble chunks: a 4x4 transpose
-// of (quarter-wave, word) -- quarter-wave 2j+rb holds rows 16rb..+15 of K-step j -- puts word q of
-// row 16rb + r into lane (r, q), register 2j+rb.  Byte chunks: quarter-wave 2c+rb holds chunk c of
-// rows 16rb..+15; swapping odd with even quarter-waves puts bytes 8q..8q+7 of the row (chunk q/2,
-// words 2(q%2), +1) into lane (r, q), registers (2rb, 2rb+1).
-template <int FMT, int NB>
-__device__ __forceinline__ void exch(const PRaw<FMT, NB> &p, ARaw<FMT, NB> (&a)[2][MF_RBW]) {
-    using P = Planes<FMT, NB>;
-    int i = 0;
-    if constexpr (P::P8) {
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const auto e = __builtin_amdgcn_permlane16_swap(p.w8[4 * j], p.w8[4 * j + 2], false, false);
-            const auto f = __builtin_amdgcn_permlane16_swap(p.w8[4 * j + 1], p.w8[4 * j + 3], false, false);
-            a[j][0].w[i] = e[0]; a[j][0].w[i + 1] = f[0];
-            a[j][1].w[i] = e[1]; a[j][1].w[i + 1] = f[1];
-        }
-        i += 2;
-    }
-    if constexpr (P::P4) {
-        const auto x = __builtin_amdgcn_permlane32_swap(p.w4[0], p.w4[2], false, false);
-        const auto y = __builtin_amdgcn_permlane32_swap(p.w4[1], p.w4[3], false, false);
-        const auto c = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false);
-        const auto d = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
-        a[0][0].w[i] = c[0]; a[0][1].w[i] = c[1]; a[1][0].w[i] = d[0]; a[1][1].w[i] = d[1];
-        i += 1;
-    }
-    if constexpr (P::P2) {
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int r = 0; r < 2; r++) a[j][r].w[i] = p.w2[2 * j + r];
-        i += 1;
-    }
-    if constexpr (P::P1) {
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int r = 0; r < 2; r++) a[j][r].w[i] = p.w1[2 * j + r];
-    }
-}
-
-__device__ __forceinline__ uint32_t sub_h2(uint32_t p, _Float16 c) {
-    mf_h2 v = __builtin_bit_cast(mf_h2, p);
-    const mf_h2 cc = {c, c};
-    v = v + cc;                                          // exact: both operands and the result are fp16 integers
-    return __builtin_bit_cast(uint32_t, v);
-}
-
-// (a & m) | o in one v_and_or_b32.  gfx9's three-operand encoding takes no literal constant and
-// reads at most one scalar register, so m comes in a scalar register and o in a vector register.
-__device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t m, uint32_t o) {
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(m), "v"(o));
-    return r;
-}
-
-// Codes of the lane's 8 elements as halves in the order {0,2,1,3,4,6,5,7}.
-template <int FMT, int NB>
-__device__ __forceinline__ mf_h8 dec_a(const ARaw<FMT, NB> &a, int q) {
-    constexpr uint32_t MAG = 0x64006400u;                // fp16 1024.0 in both halves
-    uint32_t p02, p13, p46, p57;
-    _Float16 off;
-    if constexpr (FMT == BGL_Q8G64) {
-        const uint32_t x0 = a.w[0] ^ 0x80808080u, x1 = a.w[1] ^ 0x80808080u;   // u = code + 128
-        p02 = and_or(x0, 0x00FF00FFu, MAG); p13 = and_or(x0 >> 8, 0x00FF00FFu, MAG);
-        p46 = and_or(x1, 0x00FF00FFu, MAG); p57 = and_or(x1 >> 8, 0x00FF00FFu, MAG);
-        off = (_Float16)-1152.0f;
-    } else if constexpr (FMT == BGL_QNG64) {
-        constexpr int H8 = ARaw<FMT, NB>::H8, H4 = ARaw<FMT, NB>::H4, H2 = ARaw<FMT, NB>::H2, H1 = ARaw<FMT, NB>::H1;
-        constexpr int SH4 = 8 * H8, SH2 = SH4 + 4 * H4, SH1 = SH2 + 2 * H2;
-        uint32_t u02 = 0, u13 = 0, u46 = 0, u57 = 0;
-        int i = 0;
-        if constexpr (H8) {
-            const uint32_t x0 = a.w[i] ^ 0x80808080u, x1 = a.w[i + 1] ^ 0x80808080u;
-            u02 = x0 & 0x00FF00FFu; u13 = (x0 >> 8) & 0x00FF00FFu;
-            u46 = x1 & 0x00FF00FFu; u57 = (x1 >> 8) & 0x00FF00FFu;
-            i += 2;
-        }
-        if constexpr (H4) {
-            const uint32_t w = a.w[i++];
-            u02 |= (w & 0x000F000Fu) << SH4; u13 |= ((w >> 8) & 0x000F000Fu) << SH4;
-            u46 |= ((w >> 4) & 0x000F000Fu) << SH4; u57 |= ((w >> 12) & 0x000F000Fu) << SH4;
-        }
-        if constexpr (H2) {
-            const uint32_t w = a.w[i++] >> (4 * (q & 1));   // crumbs 2(q%2) (elements 0..3) and +1 (4..7)
-            u02 |= (w & 0x00030003u) << SH2; u13 |= ((w >> 8) & 0x00030003u) << SH2;
-            u46 |= ((w >> 2) & 0x00030003u) << SH2; u57 |= ((w >> 10) & 0x00030003u) << SH2;
-        }
-        if constexpr (H1) {
-            const uint32_t w = a.w[i++] >> (2 * q);          // bits 2q (elements 0..3) and 2q+1 (4..7)
-            u02 |= (w & 0x00010001u) << SH1; u13 |= ((w >> 8) & 0x00010001u) << SH1;
-            u46 |= ((w >> 1) & 0x00010001u) << SH1; u57 |= ((w >> 9) & 0x00010001u) << SH1;
-        }
-        p02 = u02 | MAG; p13 = u13 | MAG; p46 = u46 | MAG; p57 = u57 | MAG;
-        off = (_Float16)(-(1024.0f + (float)(1 << (NB - 1))));
-    } else {
-        const uint32_t w = a.w[0];
-        p02 = and_or(w, 0x000F000Fu, MAG); p13 = and_or(w >> 8, 0x000F000Fu, MAG);
-        p46 = and_or(w >> 4, 0x000F000Fu, MAG); p57 = and_or(w >> 12, 0x000F000Fu, MAG);
-        off = (_Float16)-1032.0f;
-    }
-    mf_u4 r = {sub_h2(p02, off), sub_h2(p13, off), sub_h2(p46, off), sub_h2(p57, off)};
-    return __builtin_bit_cast(mf_h8, r);
-}
-
 // ==================================================================================== GEMM kernel
 // Task of this workgroup: the last task whose first workgroup is <= blockIdx.x (uniform).
 __device__ __forceinline__ int mf_task(const MfmaLaunch &L) {
@@ -309,7 +94,12 @@ template <int FMT, int NB> constexpr int a_words() {
 }
 // K-steps of weights a wave keeps in flight: a ring of depth/2 K-step pairs, Planes::WORDS
 // registers each.
-template <int FMT, int NB> constexpr int ring_depth() { return Planes<FMT, NB>::WORDS <= 4 ? 16 : Planes<FMT, NB>::WORDS <= 8 ? 8 : 4; }
+// (qNg64: the lane swaps of its planes want registers too; deeper rings, or this one beside 3 and 4 column
+// tiles, spilled: n = 4 at 16 columns 28672 x 4096 58.0 us with 16, 30.5 with 8)
+template <int FMT, int NB, int CT> constexpr int ring_depth() {
+    constexpr int W = Planes<FMT, NB>::WORDS;
+    return FMT == BGL_QNG64 ? (W <= 8 && CT <= 2 ? 8 : 4) : W <= 4 ? 16 : W <= 8 ? 8 : 4;
+}
 // LDS bytes per staged K-step: activation fragments (CT x hi/lo x 1 KB, + 16 B of row padding) +
 // the 4 tiles' scale words in the device layout (512 B for every format).
 constexpr int mf_step_lds(int CT) { return CT * 2048 + 16 + 512; }
@@ -344,7 +134,7 @@ __global__ __launch_bounds__(MF_WAVES * KW * 64) void k_gemm_mfma(MfmaLaunch L) 
     constexpr int SUT = 64 * SCW / 16;                             // scale uint4 per tile and unit
     // ring depth: halved with two slices (each wave runs half the split, and 16 waves share the
     // registers); at least 4 so that a unit's groups keep their parity pattern
-    constexpr int D = KW == 1 || ring_depth<FMT, NB>() == 4 ? ring_depth<FMT, NB>() : ring_depth<FMT, NB>() / 2;
+    constexpr int D = KW == 1 || ring_depth<FMT, NB, CT>() == 4 ? ring_depth<FMT, NB, CT>() : ring_depth<FMT, NB, CT>() / 2;
     static_assert(KPM % D == 0 && KPM % SPU == 0 && D % SPU == 0, "staged range must hold whole rings and units");
     __shared__ uint4 xs[KPM * XS];                                 // [step][CT][hi/lo][64 lanes], rows XS apart
     __shared__ uint4 ss[MF_TILES * UMAX * SUT];                    // [tile][unit][64 rows] scale words
@@ -603,7 +393,7 @@ __global__ __launch_bounds__(MF_WAVES * KW * 64) void k_gemm_mfma(MfmaLaunch L) 
             if constexpr (KW == 1) { bc = bnext; bnext = load_b(s + 1); }
             else bc = load_b(s);
             if (d % 2 == 0) {                                       // a new K-step pair: exchange, refill the slot
-                exch<FMT, NB>(ring[d / 2], apair);
+                exch<FMT, NB>(ring[d / 2], apair, ((s0 + s) >> 1) & 1);
                 load_w(ring[d / 2], s + D);                         // unconditional, clamped
             }
             mf_h8 A[MF_RBW];
@@ -791,8 +581,8 @@ static void launch_ct(const MfmaLaunch &L, dim3 grid, hipStream_t st) {
         hipFuncAttributes a2, a1;
         const bool ok2 = hipFuncGetAttributes(&a2, reinterpret_cast<const void *>(&k_gemm_mfma<FMT, NB, CT, 2>)) == hipSuccess;
         const bool ok1 = hipFuncGetAttributes(&a1, reinterpret_cast<const void *>(&k_gemm_mfma<FMT, NB, CT, 1>)) == hipSuccess;
-        // two slices unless they need private memory and one slice needs less
-        kw2 = ok2 && (a2.localSizeBytes == 0 || !ok1 || a2.localSizeBytes <= a1.localSizeBytes);
+        // two slices unless they need more than a few spilled registers and one slice needs less
+        kw2 = ok2 && (a2.localSizeBytes <= 32 || !ok1 || a2.localSizeBytes <= a1.localSizeBytes);
     }
     if (kw2) hipLaunchKernelGGL((k_gemm_mfma<FMT, NB, CT, 2>), grid, dim3(MF_WAVES * 2 * 64), 0, st, L);
     else hipLaunchKernelGGL((k_gemm_mfma<FMT, NB, CT, 1>), grid, dim3(MF_WAVES * 64), 0, st, L);
@@ -899,8 +689,8 @@ static int mf_reserve_fewer(bgl_ctx *c, int n, const BglDevTensor *Ts, int M) {
 // Measured, us, dot4 / here: q4g64 28672 x 4096 at 2 / 5 / 15 columns 40.2 / 28.9, 73.1 / 29.4, 153 /
 // 32.5; 4096 x 4096 14.3 / 12.3, 19.7 / 12.4, 35.8 / 13.0; 1536 x 1536 13.6 / 11.3, 17.5 / 11.7, 31.8 /
 // 12.4; q8g64 28672 x 4096 at 2 columns 41.1 / 34.9; qNg64 n = 6, 10 at 2: 54.5 / 38.8, 56.8 / 47.7.
-// qNg64 n <= 3 reads its crumbs and bits a dword at a time here: n = 3 at 2 / 4 / 8 columns 49.4 / 52.7,
-// 52.4 / 53.0, 94.1 / 53.3.  Against 64 bits the N(0, 1) products err by 1.6e-7 here, 2.9e-7 there.
+// n = 3 at 2 / 4: 49.4 / 34.9, 52.2 / 35.3.  Against 64 bits the N(0, 1) products err by 1.6e-7 here, 2.9e-7
+// there.
 // Below 16 columns the dot4 kernels also keep what they alone can run: tensors of 2 GiB and more, and
 // no-alloc calls whose K-split partials do not fit the fixed array.
 bool mfma_takes(const bgl_ctx *c, int n, const BglDevTensor *Ts, int M) {
@@ -911,7 +701,7 @@ bool mfma_takes(const bgl_ctx *c, int n, const BglDevTensor *Ts, int M) {
     for (int i = 0; i < n; i++)
         if ((double)Ts[i].ntiles * Ts[i].cpr * 1024.0 >= 2147483648.0) return false;
     if (c->fixed_base && c->fixed_used + mf_partials(c, n, Ts, M) * 4 + 256 > c->fixed_cap) return false;
-    return M >= (Ts[0].fmt == BGL_QNG64 && Ts[0].bits <= 3 ? 5 : 2);
+    return true;
 }
 
 
