@@ -199,6 +199,8 @@ struct MoeTask {
     const int *cpos;
     const int32_t *cidx;
     int ck;
+    const void *xfr;             // k_moe_m: the rows' fp16 fragments and their {exponent, non-finite} pairs
+    const int2 *xe;
     int mbx;                     // k_moe_x: token columns of records the launch's LDS holds (4 or 8)
 };
 
@@ -250,3 +252,9 @@ struct MoePair {
     int nb0;
 };
 int bgl_launch_moe_x2(const MoeTask &a, const MoeTask &b, int K, int nw, int cap, hipStream_t st);
+// ---- bgl_moe_m.hip: the gather on the matrix cores, over fragments of the rows ----
+bool bgl_moe_m_tensor(const BglDevTensor &T);
+size_t bgl_moe_frag_bytes(long rows, int K);
+void bgl_launch_moe_frag(const float *x0, int K0, int rows0, void *fr0, void *xe0, const float *x1, int K1, int rows1, void *fr1,
+                         void *xe1, hipStream_t st);
+int bgl_launch_moe_m(const MoeTask &a, const MoeTask *b, hipStream_t st);

@@ -1,6 +1,7 @@
 // bgl_moe.hip -- expert-stacked tensors and the expert-sorted MoE gather.
 //
-// One routed FFN call (moe_ffn_batched, qwen_infer.c:5238-5350, routing supplied by the caller):
+// One routed FFN call (moe_ffn_batched, qwen_infer.c:5238-5350, routing supplied by the caller), where it
+// does not run on the matrix cores (moe_m_ok, bgl_moe_m.hip):
 //   k_moe_bucket   sort the T*K (token, k) pairs by expert, stable in pair order (the reference's
 //                  bucket fill order) -> segment offsets, permutation, inverse permutation
 //   k_act_x24      exact activation digits of the T token rows, shared by every expert
@@ -28,6 +29,7 @@
     } while (0)
 
 #define MOE_MB 4            // token columns per weight pass of one tile
+#define MOE_M_AFF 3         // tokens from which affine int4 experts without shared ones run k_moe_m
 #define MOE_MAXW 8          // waves per workgroup: 512 threads leave 256 VGPRs for the widest formats
 
 static inline unsigned nblk(long n, int bs = 256) { return (unsigned)((n + bs - 1) / bs); }
@@ -488,6 +490,94 @@ extern "C" int bgl_gather_matvec_dev(bgl_ctx *c, const bgl_tensor *experts, cons
     return moe_run(c, Mt, experts, nullptr, units, 0, memo, x_dev, N, experts->T.K, (long)std::min(E, N) * Mt.tpe);
 }
 
+// Whether a routed FFN of T tokens runs k_moe_m (bgl_moe_m.hip): every tensor in a format it takes, and
+// enough work for its two fragment launches and the combine.  Measured on the DeepSeek-V2-Lite layer (64
+// experts, top 6), us, k_moe_x or k_moe_gemv / k_moe_m:
+//   with shared experts (one launch with the routed ones)  mixed formats: 2 tokens 92.4 / 100.8, 3: 119.7 /
+//     116.8, 8: 178.7 / 167.3, 64: 540.5 / 273.1; int4: 1: 48.6 / 49.2, 3: 84.4 / 63.9; affine int4: 1: 56.5 /
+//     51.3, 64: 528 / 174
+//   without                                                mixed: 8: 130.0 / 150.8, 16: 184.3 / 196.2; int4 3:
+//     58.8 / 59.5, 12: 117.4 / 104.6; affine int4: 2: 46.2 / 55.0, 3: 73.4 / 65.6; 32 experts of 2880 x 2880, top 8,
+//     mixed: 4: 210 / 238, 8: 282.7 / 276.6, 14: 404 / 297
+// (two pairs per expert is where mixed formats break even).  MXFP4 experts beside AF int4 ones stay refused,
+// and the tuning switches of k_moe_x keep it.
+static bool moe_m_ok(const bgl_ctx *c, const bgl_tensor *const (&stacks)[3], const bgl_tensor *const (&shared)[3], int T, int K) {
+    if (c->no_moe_x || c->no_mfma || c->force_tr || c->x_waves || c->moe_cap || c->moe_merge >= 0) return false;
+    bool mx = false, aff = false;
+    auto take = [&](const BglDevTensor &t) {
+        mx = mx || t.fmt == BGL_MXFP4;
+        aff = aff || t.fmt == BGL_Q4G64A;
+        return bgl_moe_m_tensor(t);
+    };
+    for (const bgl_tensor *st : stacks)
+        for (const bgl_tensor *e : st->experts)
+            if (!take(e->T)) return false;
+    for (const bgl_tensor *t : shared)
+        if (t && !take(t->T)) return false;
+    if (mx && aff) return false;
+    if (shared[0]) return aff || T >= 3;
+    return aff ? T >= MOE_M_AFF : (long)T * K >= 2l * (long)stacks[0]->experts.size();
+}
+
+// The FFN's gathers through k_moe_m: fragments of x, gate+up (routed and shared in one launch),
+// fragments of h, down (both), then the combine.  h / shh / dd / sdd: the fp32 work rows.
+static int moe_ffn_m(bgl_ctx *c, const bgl_tensor *gate, const bgl_tensor *up, const bgl_tensor *down, const bgl_tensor *sg,
+                     const bgl_tensor *su, const bgl_tensor *sd, const float *x_dev, const MoeScratch &S, int T, int K, float *h,
+                     float *shh, float *dd, float *sdd) {
+    const int H = gate->T.K, I = gate->T.N, Ish = sg ? sg->T.N : 0, P = T * K, E = (int)gate->experts.size();
+    // also what the digits of the same layer at fewer tokens take, which a caller may capture after this
+    const size_t t0 = std::min(T, MOE_M_AFF - 1), dig = 2 * 192 / 64, wide = std::max(H, Ish);
+    if (dbuf_reserve(c, c->moe_a, std::max(bgl_moe_frag_bytes(T, H), t0 * wide * dig), false) ||
+        dbuf_reserve(c, c->moe_b, std::max((size_t)T * 8, t0 * (wide / 64) * 8), false) ||
+        dbuf_reserve(c, c->moe_c, t0 * (wide / 32) * 32, false) ||
+        dbuf_reserve(c, c->moe_d, std::max(bgl_moe_frag_bytes(P, I) + bgl_moe_frag_bytes(T, Ish), t0 * K * I * dig), false) ||
+        dbuf_reserve(c, c->moe_e, std::max((size_t)(P + T) * 8, t0 * K * (I / 64) * 8), false) ||
+        dbuf_reserve(c, c->moe_f, t0 * K * (I / 32) * 32, false))
+        return bgl_last_code();
+    uint8_t *hf = (uint8_t *)c->moe_d.p, *sf = hf + bgl_moe_frag_bytes(P, I);
+    int2 *he = (int2 *)c->moe_e.p, *se = he + P;
+    int tok = prof_begin(c, 0);
+    bgl_launch_moe_frag(x_dev, H, T, c->moe_a.p, c->moe_b.p, nullptr, H, 0, nullptr, nullptr, c->stream);
+    prof_end(c, tok);
+    HIPCHK(hipGetLastError());
+    MoeTask r, s;
+    memset(&r, 0, sizeof r);
+    memset(&s, 0, sizeof s);
+    int units;
+    max_units(gate, r.tpe, units);
+    r.ta = (const BglDevTensor *)gate->dev_table; r.tb = (const BglDevTensor *)up->dev_table;
+    r.E = E; r.off = S.off; r.cols = S.tok; r.y = h; r.ystride = I; r.swiglu = 1;
+    r.xfr = c->moe_a.p; r.xe = (const int2 *)c->moe_b.p; r.a.xf = x_dev;
+    if (sg) {
+        s.da = sg->T; s.db = su->T; s.tpe = sg->T.ntiles; s.ncols = T; s.seg = 16; s.E = (T + 15) / 16;
+        s.y = shh; s.ystride = Ish; s.swiglu = 1;
+        s.xfr = r.xfr; s.xe = r.xe; s.a.xf = x_dev;
+    }
+    tok = prof_begin(c, 1);
+    bgl_launch_moe_m(r, sg ? &s : nullptr, c->stream);
+    prof_end(c, tok);
+    HIPCHK(hipGetLastError());
+    tok = prof_begin(c, 0);
+    // (pairs whose expert id was out of range leave rows past the last segment unwritten; no segment reads them)
+    bgl_launch_moe_frag(h, I, P, hf, he, shh, Ish, sg ? T : 0, sf, se, c->stream);
+    prof_end(c, tok);
+    HIPCHK(hipGetLastError());
+    memset(&r, 0, sizeof r);
+    max_units(down, r.tpe, units);
+    r.ta = (const BglDevTensor *)down->dev_table; r.E = E; r.off = S.off; r.y = dd; r.ystride = H;
+    r.xfr = hf; r.xe = he; r.a.xf = h;
+    if (sg) {
+        memset(&s, 0, sizeof s);
+        s.da = sd->T; s.tpe = sd->T.ntiles; s.ncols = T; s.seg = 16; s.E = (T + 15) / 16; s.y = sdd; s.ystride = H;
+        s.xfr = sf; s.xe = se; s.a.xf = shh;
+    }
+    tok = prof_begin(c, 1);
+    bgl_launch_moe_m(r, sg ? &s : nullptr, c->stream);
+    prof_end(c, tok);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
 // The routed FFN; pre: the pairs' bucketing when the caller already made it (the whole-layer entry).
 static int moe_ffn(bgl_ctx *c, const bgl_tensor *gate, const bgl_tensor *up, const bgl_tensor *down, const bgl_tensor *sg,
                    const bgl_tensor *su, const bgl_tensor *sd, const float *x_dev, const int32_t *idx_dev, const float *w_dev,
@@ -531,6 +621,11 @@ static int moe_ffn(bgl_ctx *c, const bgl_tensor *gate, const bgl_tensor *up, con
     if (dbuf_reserve(c, c->moe_g, (nh + nsh_h + nd + nsd) * 4, false)) return bgl_last_code();
     float *h = (float *)c->moe_g.p, *shh = h + nh, *dd = shh + nsh_h, *sdd = dd + nd;
 
+    bool combined = false;
+    const bgl_tensor *const stacks[3] = {gate, up, down}, *const shared[3] = {sg, su, sd};
+    if (moe_m_ok(c, stacks, shared, T, K)) {
+        if ((rc = moe_ffn_m(c, gate, up, down, sg, su, sd, x_dev, S, T, K, h, shh, dd, sdd))) return rc;
+    } else {
     MoeTask Mr, Ms;
     PrepMemo mx, mh, ms;                      // digits of x (slot 0), of h (slot 1), of the shared h (slot 0)
     memset(&Mr, 0, sizeof Mr);
@@ -580,7 +675,6 @@ static int moe_ffn(bgl_ctx *c, const bgl_tensor *gate, const bgl_tensor *up, con
     max_units(down, Mr.tpe, units);
     Mr.ta = (const BglDevTensor *)down->dev_table; Mr.E = E; Mr.off = S.off; Mr.y = dd; Mr.ystride = H;
     if ((rc = moe_run(c, Mr, down, nullptr, units, 1, mh, h, P, I, act_r * Mr.tpe))) return rc;
-    bool combined = false;
     if (shm) {
         if ((rc = bgl_mlp_dev(c, sg, su, sd, BGL_ACT_F32, x_dev, sdd, T, shh))) return rc;
     } else if (nsh) {
@@ -593,6 +687,7 @@ static int moe_ffn(bgl_ctx *c, const bgl_tensor *gate, const bgl_tensor *up, con
             combined = true;
         }
         if ((rc = moe_run(c, Ms, nullptr, nullptr, sd->T.nunits, 0, ms, shh, T, Ish, (long)Ms.E * Ms.tpe))) return rc;
+    }
     }
     if (combined) return 0;
     int tok = prof_begin(c, 2);
