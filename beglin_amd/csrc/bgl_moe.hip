@@ -499,7 +499,8 @@ extern "C" int bgl_gather_matvec_dev(bgl_ctx *c, const bgl_tensor *experts, cons
 //   without                                                mixed: 8: 130.0 / 150.8, 16: 184.3 / 196.2; int4 3:
 //     58.8 / 59.5, 12: 117.4 / 104.6; affine int4: 2: 46.2 / 55.0, 3: 73.4 / 65.6; 32 experts of 2880 x 2880, top 8,
 //     mixed: 4: 210 / 238, 8: 282.7 / 276.6, 14: 404 / 297
-// (two pairs per expert is where mixed formats break even).  MXFP4 experts beside AF int4 ones stay refused,
+// (two pairs per expert is where mixed formats break even; k_moe_m with 4 K slices, the 2 it has now are up
+// to 8% faster).  MXFP4 experts beside AF int4 ones stay refused,
 // and the tuning switches of k_moe_x keep it.
 static bool moe_m_ok(const bgl_ctx *c, const bgl_tensor *const (&stacks)[3], const bgl_tensor *const (&shared)[3], int T, int K) {
     if (c->no_moe_x || c->no_mfma || c->force_tr || c->x_waves || c->moe_cap || c->moe_merge >= 0) return false;

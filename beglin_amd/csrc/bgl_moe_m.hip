@@ -7,7 +7,7 @@
 // bgl_mfma.hip has the numerics: exact weights, activations to 2^-21 of themselves) and a workgroup
 // multiplies 16 tokens at a time:
 //
-//   workgroup = one 64-row tile of one expert (gate and up rows together), 8 waves = 2 row halves x 4 K
+//   workgroup = one 64-row tile of one expert (gate and up rows together), 4 waves = 2 row halves x 2 K
 //   slices.  A wave streams its 32 rows' weights straight from HBM (a pair of K-steps ahead, or two for
 //   int4), decodes them once per 16 tokens and multiplies them by the tokens' fragments, read from the
 //   L2: the rows of a segment lie anywhere, a lane reads 16 bytes of its own token's row.  Nothing is
@@ -17,14 +17,20 @@
 // loaded with the weights, and the store writes consecutive rows.  qNg64 n > 10 codes are not exact in
 // fp16 as one number: the low byte and 256 times the rest are two operands (n = 11..15).  Affine int4
 // takes codes minus 8 and adds (b + 8 s) * sum(x), the sum from two more products with ones.
-// (DeepSeek-V2-Lite mixed layer at 64 / 16 / 8 tokens: 540 -> 273, 281 -> 218, 179 -> 167 us.)
+// (DeepSeek-V2-Lite mixed layer at 64 / 8 tokens: 548 -> 242, 179 -> 154 us; affine int4 at 16 218 -> 125.)
+//
+// What bounds it: the weights' arrival at 12 waves per CU (mixed layer at 64 tokens: 3.0 TB/s over all seven
+// launches).  3 waves per SIMD leave 168 registers, where 4 of the widest formats' gate+up spill; at 4 waves
+// (128 registers) 89 did.  2 x 4 slices at 4 waves: 272 us at 64 tokens, 161 at 8, affine int4 at 16 123; 2 x 2
+// at 4 waves 278, 167, 117; 2 x 2 at 3 waves 249, 149, 116.  (8 waves a workgroup fit a CU at 3 per SIMD only
+// once.)  Sending the first weights out before the token's row number is known changed nothing (272, 162, 124).
 #include <string.h>
 
 #include "bgl_internal.h"
 #include "bgl_mfma_a.h"
 
 #define MM_COLS 16               // tokens per pass over the weights
-#define MM_KS 4                  // K slices (waves) per row half
+#define MM_KS 2                  // K slices (waves) per row half
 #define MM_WAVES (2 * MM_KS)
 
 // ------------------------------------------------------------------ activation fragments
@@ -321,7 +327,7 @@ __device__ __forceinline__ BglDevTensor mm_tensor(const BglDevTensor *p) {
 }
 
 template <bool GLU>
-__global__ __launch_bounds__(MM_WAVES * 64, 4) void k_moe_m(MoePair P) {
+__global__ __launch_bounds__(MM_WAVES * 64, 3) void k_moe_m(MoePair P) {
     __shared__ float red[MM_KS * (GLU ? 2 : 1) * 1024];
     const int second = (int)blockIdx.x >= P.nb0, b = second ? (int)blockIdx.x - P.nb0 : (int)blockIdx.x;
     MoeTask Mt = P.t[0];

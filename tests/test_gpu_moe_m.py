@@ -45,7 +45,7 @@ def test_moe_m_formats(ctx, torch_dev, oracle, fmt):  # noqa: F811
 
 @pytest.mark.parametrize("T,K,Ish", [(3, 2, 64), (16, 1, 0), (17, 3, 0), (64, 2, 128)])
 def test_moe_m_shapes(ctx, torch_dev, oracle, T, K, Ish):  # noqa: F811
-    """Mixed formats; one 64-group per row (three of the four slices empty)."""
+    """Mixed formats; one 64-group per row (all K slices but the first empty)."""
     say("moe_m shapes", T, K, Ish)
     E, H, I = 4, 64, 64
     rng = np.random.default_rng(T)
