@@ -335,15 +335,22 @@ static int moe_bucket(bgl_ctx *c, const int32_t *idx_dev, int P, int K, int E, M
     return 0;
 }
 
+// The scratch of the exact activation digits of M rows of length K in digit slot 0 or 1.
+static int moe_digits(bgl_ctx *c, int slot, size_t M, int K) {
+    DevBuf &w = slot ? c->moe_d : c->moe_a, &s = slot ? c->moe_e : c->moe_b, &d = slot ? c->moe_f : c->moe_c;
+    const size_t ng = K / 64;
+    if (dbuf_reserve(c, w, 2 * M * ng * 192, false) || dbuf_reserve(c, s, 2 * M * ng * 4, false) ||
+        dbuf_reserve(c, d, 2 * M * (K / 32) * 16, false))
+        return bgl_last_code();
+    return 0;
+}
+
 // Exact activation digits of M rows of length K into digit slot 0 or 1.
 static int moe_prep(bgl_ctx *c, int slot, const float *x_dev, int M, int K, GemvAct &A) {
-    DevBuf &w = slot ? c->moe_d : c->moe_a;
-    DevBuf &s = slot ? c->moe_e : c->moe_b;
-    DevBuf &d = slot ? c->moe_f : c->moe_c;
+    const int rc = moe_digits(c, slot, M, K);
+    if (rc) return rc;
+    DevBuf &w = slot ? c->moe_d : c->moe_a, &s = slot ? c->moe_e : c->moe_b, &d = slot ? c->moe_f : c->moe_c;
     const int ng = K / 64;
-    if (dbuf_reserve(c, w, (size_t)2 * M * ng * 192, false) || dbuf_reserve(c, s, (size_t)2 * M * ng * 4, false) ||
-        dbuf_reserve(c, d, (size_t)2 * M * (K / 32) * 16, false))
-        return bgl_last_code();
     int tok = prof_begin(c, 0);
     hipLaunchKernelGGL(k_act_x24, dim3(nblk((long)M * ng * 64)), dim3(256), 0, c->stream, x_dev, M, K, (int8_t *)w.p,
                        (float *)s.p, (int *)d.p, (const float *)nullptr, (float *)nullptr);
@@ -502,6 +509,11 @@ extern "C" int bgl_gather_matvec_dev(bgl_ctx *c, const bgl_tensor *experts, cons
 // (two pairs per expert is where mixed formats break even; k_moe_m with 4 K slices, the 2 it has now are up
 // to 8% faster).  MXFP4 experts beside AF int4 ones stay refused,
 // and the tuning switches of k_moe_x keep it.
+// moe_m_below: the most tokens that stay with the other gathers (aff: an affine int4 tensor among them).
+static int moe_m_below(const bgl_tensor *const (&stacks)[3], const bgl_tensor *const (&shared)[3], bool aff, int K) {
+    if (shared[0]) return aff ? 0 : 2;
+    return aff ? MOE_M_AFF - 1 : (2 * (int)stacks[0]->experts.size() - 1) / K;
+}
 static bool moe_m_ok(const bgl_ctx *c, const bgl_tensor *const (&stacks)[3], const bgl_tensor *const (&shared)[3], int T, int K) {
     if (c->no_moe_x || c->no_mfma || c->force_tr || c->x_waves || c->moe_cap || c->moe_merge >= 0) return false;
     bool mx = false, aff = false;
@@ -516,8 +528,34 @@ static bool moe_m_ok(const bgl_ctx *c, const bgl_tensor *const (&stacks)[3], con
     for (const bgl_tensor *t : shared)
         if (t && !take(t->T)) return false;
     if (mx && aff) return false;
-    if (shared[0]) return aff || T >= 3;
-    return aff ? T >= MOE_M_AFF : (long)T * K >= 2l * (long)stacks[0]->experts.size();
+    return T > moe_m_below(stacks, shared, aff, K);
+}
+
+// The digits of the same layer at fewer tokens, which a caller may capture once this call has run: only
+// where those tokens stay with the other gathers and k_moe_x does not take their launches (affine int4,
+// or a width whose records do not fit its LDS).
+static int moe_digits_fewer(bgl_ctx *c, const bgl_tensor *const (&stacks)[3], const bgl_tensor *const (&shared)[3], int K) {
+    bool aff = false;
+    for (const bgl_tensor *st : stacks)
+        for (const bgl_tensor *e : st->experts) aff = aff || e->T.fmt == BGL_Q4G64A;
+    for (const bgl_tensor *t : shared) aff = aff || (t && t->T.fmt == BGL_Q4G64A);
+    const int t0 = moe_m_below(stacks, shared, aff, K), H = stacks[0]->T.K, I = stacks[0]->T.N;
+    if (t0 < 1) return 0;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    HIPCHK(hipStreamIsCapturing(c->stream, &cs));
+    if (cs != hipStreamCaptureStatusNone) return 0;                // this call does without them
+    MoeTask r, s;
+    memset(&r, 0, sizeof r);
+    memset(&s, 0, sizeof s);
+    r.ta = (const BglDevTensor *)stacks[0]->dev_table;             // (not the by-value tensors)
+    const bool sh = shared[0] != nullptr;
+    if (sh) { s.da = shared[0]->T; s.db = shared[1]->T; s.swiglu = 1; }
+    if (!moe_x_ok(c, stacks[0], stacks[1], r, H) || (sh && !moe_x_ok(c, nullptr, nullptr, s, H)))
+        if (moe_digits(c, 0, t0, H)) return bgl_last_code();
+    if (!moe_x_ok(c, stacks[2], nullptr, r, I) && moe_digits(c, 1, (size_t)t0 * K, I)) return bgl_last_code();
+    if (sh) { s.da = shared[2]->T; s.swiglu = 0; }
+    if (sh && !moe_x_ok(c, nullptr, nullptr, s, shared[2]->T.K) && moe_digits(c, 0, t0, shared[2]->T.K)) return bgl_last_code();
+    return 0;
 }
 
 // The FFN's gathers through k_moe_m: fragments of x, gate+up (routed and shared in one launch),
@@ -526,14 +564,9 @@ static int moe_ffn_m(bgl_ctx *c, const bgl_tensor *gate, const bgl_tensor *up, c
                      const bgl_tensor *su, const bgl_tensor *sd, const float *x_dev, const MoeScratch &S, int T, int K, float *h,
                      float *shh, float *dd, float *sdd) {
     const int H = gate->T.K, I = gate->T.N, Ish = sg ? sg->T.N : 0, P = T * K, E = (int)gate->experts.size();
-    // also what the digits of the same layer at fewer tokens take, which a caller may capture after this
-    const size_t t0 = std::min(T, MOE_M_AFF - 1), dig = 2 * 192 / 64, wide = std::max(H, Ish);
-    if (dbuf_reserve(c, c->moe_a, std::max(bgl_moe_frag_bytes(T, H), t0 * wide * dig), false) ||
-        dbuf_reserve(c, c->moe_b, std::max((size_t)T * 8, t0 * (wide / 64) * 8), false) ||
-        dbuf_reserve(c, c->moe_c, t0 * (wide / 32) * 32, false) ||
-        dbuf_reserve(c, c->moe_d, std::max(bgl_moe_frag_bytes(P, I) + bgl_moe_frag_bytes(T, Ish), t0 * K * I * dig), false) ||
-        dbuf_reserve(c, c->moe_e, std::max((size_t)(P + T) * 8, t0 * K * (I / 64) * 8), false) ||
-        dbuf_reserve(c, c->moe_f, t0 * K * (I / 32) * 32, false))
+    if (dbuf_reserve(c, c->moe_a, bgl_moe_frag_bytes(T, H), false) || dbuf_reserve(c, c->moe_b, (size_t)T * 8, false) ||
+        dbuf_reserve(c, c->moe_d, bgl_moe_frag_bytes(P, I) + bgl_moe_frag_bytes(T, Ish), false) ||
+        dbuf_reserve(c, c->moe_e, (size_t)(P + T) * 8, false))
         return bgl_last_code();
     uint8_t *hf = (uint8_t *)c->moe_d.p, *sf = hf + bgl_moe_frag_bytes(P, I);
     int2 *he = (int2 *)c->moe_e.p, *se = he + P;
@@ -625,6 +658,7 @@ static int moe_ffn(bgl_ctx *c, const bgl_tensor *gate, const bgl_tensor *up, con
     bool combined = false;
     const bgl_tensor *const stacks[3] = {gate, up, down}, *const shared[3] = {sg, su, sd};
     if (moe_m_ok(c, stacks, shared, T, K)) {
+        if ((rc = moe_digits_fewer(c, stacks, shared, K))) return rc;
         if ((rc = moe_ffn_m(c, gate, up, down, sg, su, sd, x_dev, S, T, K, h, shh, dd, sdd))) return rc;
     } else {
     MoeTask Mr, Ms;

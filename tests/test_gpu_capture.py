@@ -13,6 +13,7 @@ import numpy as np
 import pytest
 
 from golden.fixtures import seeded_normal
+from oracle_ffi import moe_ffn
 
 pytestmark = pytest.mark.gpu
 
@@ -143,4 +144,58 @@ def test_capture_that_needs_more_scratch_is_refused(torch_dev, oracle):
     got = y8.cpu().numpy()
     assert np.max(np.abs(got - ref)) / np.max(np.abs(ref)) <= 1e-5
     t.free()
+    c.close()
+
+
+@pytest.mark.parametrize("H,I,fm,Ish", [(192, 9216, (5, 9), 0), (9216, 192, (5, 9), 0), (320, 256, (6,), 0), (9216, 192, (5, 9), 64)])
+def test_routed_capture_at_fewer_tokens(torch_dev, oracle, H, I, fm, Ish):
+    """A routed layer that ran at 16 tokens (matrix cores) may be captured at any fewer, also where the
+    fewer tokens take another gather, whose prepared digits a width past 9k or affine int4 experts need."""
+    import beglin_amd
+    torch = torch_dev
+    E, K = 8, 2
+    s = torch.cuda.Stream()
+    c = beglin_amd.Context(0, stream=s.cuda_stream)
+
+    def desc(e, o, i, seed):
+        f = fm[e % len(fm)]
+        if f == 6:
+            rng = np.random.default_rng(seed)
+            return (6, 4, rng.integers(0, 256, (o, i // 2), dtype=np.uint8), rng.random((o, i // 64), dtype=np.float32) * np.float32(0.01),
+                    rng.standard_normal((o, i // 64), dtype=np.float32) * np.float32(0.04))
+        w = seeded_normal(seed, (o, i), 0.02)
+        return (5, 0, *oracle.quantize_q4g32h(w)) if f == 5 else (4, 9, *oracle.quantize_qng64(w, 9))
+
+    gate, up, down = ([desc(e, o, i, 700 + 100 * j + e) for e in range(E)] for j, (o, i) in enumerate(((I, H), (I, H), (H, I))))
+    stacks = [c.bind_experts(d) for d in (gate, up, down)]
+    shared = sh = None
+    if Ish:
+        shared = tuple((5, 0, *oracle.quantize_q4g32h(seeded_normal(1000 + j, oi, 0.02))) for j, oi in enumerate(((Ish, H), (Ish, H), (H, Ish))))
+        sh = tuple(c.bind(5, d[2], d[3], d[2].shape[0], d[2].shape[1] * 2) for d in shared)
+    x = seeded_normal(1010, (16, H))
+    idx, w = oracle.route(seeded_normal(1011, (16, E)), K, True)
+    ref = moe_ffn(oracle, gate, up, down, shared, H, I, x, idx, w)
+    xd, idxd, wd = dev(torch, x), dev(torch, idx), dev(torch, w)
+    y = torch.zeros((16, H), device="cuda")
+    torch.cuda.synchronize()
+    c.moe_ffn(*stacks, sh, xd, idxd, wd, y)
+    c.sync()
+    for T in (16, 7, 3, 2, 1):
+        say("routed capture", H, I, fm, Ish, T)
+        yt = torch.zeros((T, H), device="cuda")
+        xt, it, wt = xd[:T].contiguous(), idxd[:T].contiguous(), wd[:T].contiguous()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            c.moe_ffn(*stacks, sh, xt, it, wt, yt)
+        for _ in range(2):
+            yt.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            got = yt.cpu().numpy()
+            assert np.max(np.abs(got - ref[:T])) / np.max(np.abs(ref[:T])) <= 1e-5, T
+        del graph
+    for t in stacks + list(sh or ()):
+        t.free()
     c.close()
