@@ -558,20 +558,22 @@ static int moe_digits_fewer(bgl_ctx *c, const bgl_tensor *const (&stacks)[3], co
     return 0;
 }
 
+// Bytes of the fragments and row exponents of a call, in one allocation with its fp32 rows (a context's
+// first call pays for each).
+static size_t moe_m_bytes(int T, int P, int H, int I, int Ish) {
+    return bgl_moe_frag_bytes(T, H) + bgl_moe_frag_bytes(P, I) + bgl_moe_frag_bytes(T, Ish) + (size_t)(2 * T + P) * sizeof(int2);
+}
+
 // The FFN's gathers through k_moe_m: fragments of x, gate+up (routed and shared in one launch),
-// fragments of h, down (both), then the combine.  h / shh / dd / sdd: the fp32 work rows.
+// fragments of h, down (both), then the combine.  h / shh / dd / sdd: the fp32 work rows; fr: moe_m_bytes.
 static int moe_ffn_m(bgl_ctx *c, const bgl_tensor *gate, const bgl_tensor *up, const bgl_tensor *down, const bgl_tensor *sg,
                      const bgl_tensor *su, const bgl_tensor *sd, const float *x_dev, const MoeScratch &S, int T, int K, float *h,
-                     float *shh, float *dd, float *sdd) {
+                     float *shh, float *dd, float *sdd, uint8_t *fr) {
     const int H = gate->T.K, I = gate->T.N, Ish = sg ? sg->T.N : 0, P = T * K, E = (int)gate->experts.size();
-    if (dbuf_reserve(c, c->moe_a, bgl_moe_frag_bytes(T, H), false) || dbuf_reserve(c, c->moe_b, (size_t)T * 8, false) ||
-        dbuf_reserve(c, c->moe_d, bgl_moe_frag_bytes(P, I) + bgl_moe_frag_bytes(T, Ish), false) ||
-        dbuf_reserve(c, c->moe_e, (size_t)(P + T) * 8, false))
-        return bgl_last_code();
-    uint8_t *hf = (uint8_t *)c->moe_d.p, *sf = hf + bgl_moe_frag_bytes(P, I);
-    int2 *he = (int2 *)c->moe_e.p, *se = he + P;
+    uint8_t *xf = fr, *hf = xf + bgl_moe_frag_bytes(T, H), *sf = hf + bgl_moe_frag_bytes(P, I);
+    int2 *xe = (int2 *)(sf + bgl_moe_frag_bytes(T, Ish)), *he = xe + T, *se = he + P;
     int tok = prof_begin(c, 0);
-    bgl_launch_moe_frag(x_dev, H, T, c->moe_a.p, c->moe_b.p, nullptr, H, 0, nullptr, nullptr, c->stream);
+    bgl_launch_moe_frag(x_dev, H, T, xf, xe, nullptr, H, 0, nullptr, nullptr, c->stream);
     prof_end(c, tok);
     HIPCHK(hipGetLastError());
     MoeTask r, s;
@@ -581,7 +583,7 @@ static int moe_ffn_m(bgl_ctx *c, const bgl_tensor *gate, const bgl_tensor *up, c
     max_units(gate, r.tpe, units);
     r.ta = (const BglDevTensor *)gate->dev_table; r.tb = (const BglDevTensor *)up->dev_table;
     r.E = E; r.off = S.off; r.cols = S.tok; r.y = h; r.ystride = I; r.swiglu = 1;
-    r.xfr = c->moe_a.p; r.xe = (const int2 *)c->moe_b.p; r.a.xf = x_dev;
+    r.xfr = xf; r.xe = xe; r.a.xf = x_dev;
     if (sg) {
         s.da = sg->T; s.db = su->T; s.tpe = sg->T.ntiles; s.ncols = T; s.seg = 16; s.E = (T + 15) / 16;
         s.y = shh; s.ystride = Ish; s.swiglu = 1;
@@ -652,14 +654,16 @@ static int moe_ffn(bgl_ctx *c, const bgl_tensor *gate, const bgl_tensor *up, con
     else if ((rc = moe_bucket(c, idx_dev, P, K, E, S))) return rc;
     // fp32 work rows: h [P][I], shared h [T][Ish], routed down [P][H], shared down [T][H]
     const size_t nh = (size_t)P * I, nsh_h = (size_t)T * Ish, nd = (size_t)P * H, nsd = (size_t)T * H;
-    if (dbuf_reserve(c, c->moe_g, (nh + nsh_h + nd + nsd) * 4, false)) return bgl_last_code();
+    const bgl_tensor *const stacks[3] = {gate, up, down}, *const shared[3] = {sg, su, sd};
+    const bool mm = moe_m_ok(c, stacks, shared, T, K);
+    const size_t rows = (nh + nsh_h + nd + nsd) * 4;          // whole 64-groups: the fragments behind them stay aligned
+    if (dbuf_reserve(c, c->moe_g, rows + (mm ? moe_m_bytes(T, P, H, I, Ish) : 0), false)) return bgl_last_code();
     float *h = (float *)c->moe_g.p, *shh = h + nh, *dd = shh + nsh_h, *sdd = dd + nd;
 
     bool combined = false;
-    const bgl_tensor *const stacks[3] = {gate, up, down}, *const shared[3] = {sg, su, sd};
-    if (moe_m_ok(c, stacks, shared, T, K)) {
+    if (mm) {
         if ((rc = moe_digits_fewer(c, stacks, shared, K))) return rc;
-        if ((rc = moe_ffn_m(c, gate, up, down, sg, su, sd, x_dev, S, T, K, h, shh, dd, sdd))) return rc;
+        if ((rc = moe_ffn_m(c, gate, up, down, sg, su, sd, x_dev, S, T, K, h, shh, dd, sdd, (uint8_t *)c->moe_g.p + rows))) return rc;
     } else {
     MoeTask Mr, Ms;
     PrepMemo mx, mh, ms;                      // digits of x (slot 0), of h (slot 1), of the shared h (slot 0)
