@@ -83,6 +83,16 @@ int dbuf_reserve(bgl_ctx *c, DevBuf &b, size_t bytes, bool zero) {
     return 0;
 }
 
+int dbuf_grow_kept(bgl_ctx *c, DevBuf &b, size_t bytes) {
+    const DevBuf old = b;
+    if (dbuf_reserve(c, b, bytes, false)) {
+        c->prep_reuse = false;
+        return bgl_last_code();
+    }
+    if (c->prep_reuse && old.p && b.p != old.p) HIPCHK(hipMemcpyAsync(b.p, old.p, old.bytes, hipMemcpyDeviceToDevice, c->stream));
+    return 0;
+}
+
 static void dbuf_free(DevBuf &b) {
     if (b.p) (void)hipFree(b.p);
     b.p = nullptr; b.bytes = 0;
@@ -747,7 +757,6 @@ static void fill_tasks(GemvLaunch &L, int n, const BglDevTensor *Ts, const float
 }
 
 #define BGL_GEMV_X_LDS_MAX (160 * 1024)
-#define BGL_GEMV_X_FUSE_MAX_K 4096            // longer K: one prep kernel beats every workgroup making the digits
 
 // One fp32-activation column through k_gemv_x (bgl_gemv_x.hip): workgroups of TR rows over the whole
 // K range, waves taking slots of 64/TR groups in turn, so no launch needs a K split.  A: the prepared
@@ -1002,7 +1011,7 @@ int run_down_swiglu_w4a8(bgl_ctx *c, const BglDevTensor &down, const float *g, c
 int run_down_swiglu_f32(bgl_ctx *c, const bgl_tensor *down, const float *g, const float *u, float *h, int M, float *y) {
     const BglDevTensor &T = down->T;
     if (mfma_takes(c, 1, &T, M) || !(gemv_x_kind(T.fmt))) return 1;
-    if (M == 1 && !c->no_gemv_x && (c->x_fuse == 1 || (c->x_fuse < 0 && T.K <= BGL_GEMV_X_FUSE_MAX_K))) return 1;
+    if (M == 1 && gemv_x_fuses(c, T.K)) return 1;
     c->prep_u = u;
     c->prep_h = h;
     const int rc = bgl_matmul_dev(c, down, BGL_ACT_F32, g, nullptr, y, M);
@@ -1041,8 +1050,7 @@ extern "C" int bgl_matmul_group_dev(bgl_ctx *c, int n, const bgl_tensor *const *
     if (act == BGL_ACT_W4A8 && fused_q_ok(c, kind, Ts[0].K, M)) return run_gemv_q(c, n, Ts, x_dev, M, bias_dev, y_dev);
     if (act == BGL_ACT_F32 && mfma_takes(c, n, Ts, M)) return run_gemm_mfma(c, n, Ts, x_dev, M, bias_dev, y_dev, nullptr);
     // one fp32 column over a short K: the GEMV makes the activation digits itself (no prep launch)
-    if (act == BGL_ACT_F32 && M == 1 && !c->no_gemv_x && gemv_x_kind(kind) &&
-        (c->x_fuse == 1 || (c->x_fuse < 0 && Ts[0].K <= BGL_GEMV_X_FUSE_MAX_K))) {
+    if (act == BGL_ACT_F32 && M == 1 && gemv_x_kind(kind) && gemv_x_fuses(c, Ts[0].K)) {
         int rc = run_gemv_x(c, n, Ts, nullptr, x_dev, bias_dev, y_dev, nullptr);
         if (rc <= 0) return rc;
     }

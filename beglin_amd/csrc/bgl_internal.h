@@ -83,6 +83,8 @@ bgl_tensor *tensor_from_parts(const BglDevTensor &T, void *w, void *s0, void *s1
 int prof_begin(bgl_ctx *c, int phase);
 void prof_end(bgl_ctx *c, int token);
 int dbuf_reserve(bgl_ctx *c, DevBuf &b, size_t bytes, bool zero);
+// The same for act_w / act_s / act_sum, whose prepared operands (prep_reuse) are copied along.
+int dbuf_grow_kept(bgl_ctx *c, DevBuf &b, size_t bytes);
 // Bytes of per-call scratch the context holds; with release, frees it (the caller synchronizes).
 size_t ctx_scratch(bgl_ctx *c, bool release);
 int check_wt(int kind, int bits, int out, int in);
@@ -94,6 +96,12 @@ int run_gemv(bgl_ctx *c, int n, const BglDevTensor *Ts, int act, const GemvAct &
 // Batched fp32-activation GEMM on the matrix cores (bgl_mfma.hip): formats it takes, and the call.
 #define BGL_MFMA_MIN_M 16               // the routed FFN's shared experts leave the gather from this many tokens
 bool bgl_mfma_ok(int fmt, int bits);
+// Whether one fp32 column over K makes its digits inside the GEMV (longer K: one prep kernel beats every
+// workgroup making them).
+#define BGL_GEMV_X_FUSE_MAX_K 4096
+static inline bool gemv_x_fuses(const bgl_ctx *c, int K) {
+    return !c->no_gemv_x && (c->x_fuse == 1 || (c->x_fuse < 0 && K <= BGL_GEMV_X_FUSE_MAX_K));
+}
 // Whether a group's products of M fp32 columns run there.
 bool mfma_takes(const bgl_ctx *c, int n, const BglDevTensor *Ts, int M);
 // glu_h (n == 2, a gate/up pair of one shape): the reduce launch also forms h = silu(gate) * up

@@ -658,29 +658,31 @@ static size_t mf_partials(const bgl_ctx *c, int n, const BglDevTensor *Ts, int M
 }
 
 // Scratch for the same call at fewer columns, which a caller may capture once this one has run: the
-// partials do not grow strictly with the columns (this bounds them), and the fewest columns take the
-// digits of k_act_x24.
+// partials do not grow strictly with the columns (this bounds them), and one column over a long K takes
+// the digits of k_act_x24.  Operands that bgl_prep_act_dev left in the digits' buffers move with them.
 static int mf_reserve_fewer(bgl_ctx *c, int n, const BglDevTensor *Ts, int M) {
     const int Mc = std::min(M, 16 * MF_MAXCT), CT = (Mc + 15) / 16;
     const int kpm = CT == 1 ? mf_kps_max(1) : CT == 2 ? mf_kps_max(2) : CT == 3 ? mf_kps_max(3) : mf_kps_max(4);
-    const size_t ng = Ts[0].K / 64, md = std::min(M, 4);
+    const size_t ng = Ts[0].K / 64;
     double fl = 0.0;
     for (int i = 0; i < n; i++) {
         const int wgr = (Ts[i].ntiles + MF_TILES - 1) / MF_TILES, smin = (Ts[i].K / 32 + kpm - 1) / kpm;
         const double most = std::min((double)((c->min_blocks + wgr - 1) / wgr) * Mc * Ts[i].N, c->mf_pcap * mf_weight_bytes(Ts[i]) / 8.0);
         fl += std::max(most, smin > 1 ? (double)smin * Mc * Ts[i].N : 0.0);
     }
-    const size_t pb = (size_t)fl * 4, db = 2 * md * ng * 192;
-    // operands that bgl_prep_act_dev left stay where they are
-    const bool dig = !c->prep_reuse;
-    if (c->part.bytes >= pb && (!dig || (c->act_w.bytes >= db && c->act_s.bytes >= 2 * md * ng * 4 && c->act_sum.bytes >= 4 * md * ng * 16))) return 0;
+    const size_t pb = (size_t)fl * 4;
+    const bool dig = !gemv_x_fuses(c, Ts[0].K) || Ts[0].K > BGL_GEMV_X_FUSE_MAX_K;
+    const struct { DevBuf *b; size_t bytes; } need[3] = {{&c->act_w, 2 * ng * 192}, {&c->act_s, 2 * ng * 4}, {&c->act_sum, 4 * ng * 16}};
+    bool have = c->part.bytes >= pb;
+    for (auto &d : need) have = have && (!dig || d.b->bytes >= d.bytes);
+    if (have) return 0;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     HIPCHK(hipStreamIsCapturing(c->stream, &cs));
     if (cs != hipStreamCaptureStatusNone) return 0;                // this call may still have all that it needs
     if (dbuf_reserve(c, c->part, pb, false)) return bgl_last_code();
-    if (dig && (dbuf_reserve(c, c->act_w, db, false) || dbuf_reserve(c, c->act_s, 2 * md * ng * 4, false) ||
-                dbuf_reserve(c, c->act_sum, 4 * md * ng * 16, false)))
-        return bgl_last_code();
+    if (dig)
+        for (auto &d : need)
+            if (dbuf_grow_kept(c, *d.b, d.bytes)) return bgl_last_code();
     return 0;
 }
 

@@ -199,3 +199,46 @@ def test_routed_capture_at_fewer_tokens(torch_dev, oracle, H, I, fm, Ish):
     for t in stacks + list(sh or ()):
         t.free()
     c.close()
+
+
+@pytest.mark.parametrize("kind,pre", [(1, 0), (4, 0), (1, 1)])
+def test_one_column_captured_after_several_and_a_prep(torch_dev, oracle, kind, pre):
+    """Operands prepared for another product (bgl_prep_act_dev) are in the context when a call of several
+    columns runs: a capture of that call at one column, which needs prepared digits (K > 4096), still
+    works, and the prepared operands are still the ones that were prepared."""
+    import beglin_amd
+    torch = torch_dev
+    say("one column after a prep", kind, pre)
+    s = torch.cuda.Stream()
+    c = beglin_amd.Context(0, stream=s.cuda_stream)
+    N, K = 96, 8192
+    w = seeded_normal(520, (N, K), 0.02)
+    p, sc = oracle.quantize_qng64(w, 6) if kind == 4 else oracle.quantize_q4g64(w)
+    t = c.bind(kind, p, sc, N, K, bits=6 if kind == 4 else 0)
+    pp, ps = oracle.quantize_q4g64(seeded_normal(521, (80, 512), 0.02))
+    tp = c.bind(1, pp, ps, 80, 512)
+    x, xp = seeded_normal(522, (5, K)), seeded_normal(523, (3, 512))
+    xd, xpd = dev(torch, x), dev(torch, xp)
+    y, yp = torch.zeros((5, N), device="cuda"), torch.zeros((3, 80), device="cuda")
+    torch.cuda.synchronize()
+    c.prep_only(xpd, pre, tp)
+    c.matmul(t, xd, y)
+    c.sync()
+    y1 = torch.zeros((1, N), device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    c.matmul_prepped(tp, yp, act=pre, M=3)                # before the capture, which prepares its own
+    with torch.cuda.graph(graph, stream=s):
+        c.matmul(t, xd[:1], y1)
+    ref = oracle.gemm_f32(kind, p, sc, x[:1], bits=6 if kind == 4 else 0)
+    for _ in range(2):
+        y1.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.max(np.abs(y1.cpu().numpy() - ref)) / np.max(np.abs(ref)) <= 1e-5
+    refp = oracle.gemm_f32(1, pp, ps, xp) if pre == 0 else oracle.matmul_sdot(1, pp, ps, xp)
+    assert np.max(np.abs(yp.cpu().numpy() - refp)) / np.max(np.abs(refp)) <= 1e-5
+    for q in (t, tp):
+        q.free()
+    c.close()
