@@ -83,13 +83,22 @@ int dbuf_reserve(bgl_ctx *c, DevBuf &b, size_t bytes, bool zero) {
     return 0;
 }
 
-int dbuf_grow_kept(bgl_ctx *c, DevBuf &b, size_t bytes) {
-    const DevBuf old = b;
-    if (dbuf_reserve(c, b, bytes, false)) {
-        c->prep_reuse = false;
-        return bgl_last_code();
+int act_reserve_fewer(bgl_ctx *c, size_t w, size_t s, size_t sum) {
+    DevBuf *const bufs[3] = {&c->act_w, &c->act_s, &c->act_sum};
+    const size_t bytes[3] = {w, s, sum};
+    if (c->act_w.bytes >= w && c->act_s.bytes >= s && c->act_sum.bytes >= sum) return 0;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    HIPCHK(hipStreamIsCapturing(c->stream, &cs));
+    if (cs != hipStreamCaptureStatusNone) return 0;
+    for (int i = 0; i < 3; i++) {
+        const DevBuf old = *bufs[i];
+        if (dbuf_reserve(c, *bufs[i], bytes[i], false)) {
+            c->prep_reuse = false;
+            return bgl_last_code();
+        }
+        if (c->prep_reuse && old.p && bufs[i]->p != old.p)
+            HIPCHK(hipMemcpyAsync(bufs[i]->p, old.p, old.bytes, hipMemcpyDeviceToDevice, c->stream));
     }
-    if (c->prep_reuse && old.p && b.p != old.p) HIPCHK(hipMemcpyAsync(b.p, old.p, old.bytes, hipMemcpyDeviceToDevice, c->stream));
     return 0;
 }
 

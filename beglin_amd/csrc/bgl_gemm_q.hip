@@ -407,21 +407,21 @@ int run_gemm_q(bgl_ctx *c, int n, const BglDevTensor *Ts, const float *x_dev, co
                const float *const *bias, float *const *y) {
     const int K = Ts[0].K, fmt = Ts[0].fmt, gq = fmt == BGL_Q4G256SF ? 256 : 64;
     const int mc0 = std::min(M, GQ_COLS), cbm = (mc0 + 31) / 32;
-    // (act_sum is not used here: the same call at fewer columns may take it, inside a capture)
-    if (dbuf_reserve(c, c->act_w, (size_t)32 * cbm * K, false) ||
-        dbuf_reserve(c, c->act_s, (size_t)GQ_COLS * ((K / gq + 3) / 4 * 4) * 4, false) ||
-        (!c->fixed_base && dbuf_reserve(c, c->act_sum, (size_t)std::min(M, 16) * (K / 64) * 4, false)))
-        return bgl_last_code();
-    c->prep_act = -1;                                             // the prepared-activation state is overwritten
-    c->prep_reuse = false;
-    c->prep_x = nullptr;
+    // The codes and scales lie in the partials' buffer, which no call leaves anything in: operands that
+    // bgl_prep_act_dev left stay.  The same call at fewer columns prepares its own, possibly in a capture.
+    const size_t xb = (size_t)32 * cbm * K, sb = (size_t)GQ_COLS * ((K / gq + 3) / 4 * 4) * 4;   // (xb: a multiple of 2048)
+    if (dbuf_reserve(c, c->part, xb + sb, false)) return bgl_last_code();
+    const size_t few = std::min(M, 16);
+    if (!c->fixed_base && act_reserve_fewer(c, few * K, few * (K / gq) * 4, few * (K / 64) * 4)) return bgl_last_code();
+    uint8_t *const xt = (uint8_t *)c->part.p;
+    float *const as = (float *)(xt + xb);
     for (int m0 = 0; m0 < M; m0 += GQ_COLS) {
         const int mc = std::min(GQ_COLS, M - m0);
         GemmQLaunch L;
         memset(&L, 0, sizeof L);
         L.cb32 = (mc + 31) / 32;
-        L.xt = (const uint8_t *)c->act_w.p;
-        L.as = (const float *)c->act_s.p;
+        L.xt = xt;
+        L.as = as;
         L.m0 = m0;
         L.mcols = mc;
         L.ntasks = n;
@@ -437,11 +437,11 @@ int run_gemm_q(bgl_ctx *c, int n, const BglDevTensor *Ts, const float *x_dev, co
         const unsigned pb = (unsigned)(((long)mc * ((K + 255) / 256) + 3) / 4);
         int tok = prof_begin(c, 0);
         if (gq == 256)
-            hipLaunchKernelGGL((k_act_q_tiles<256>), dim3(pb), dim3(256), 0, c->stream, x_dev + xo, mc, K, L.cb32, split, am, (uint8_t *)c->act_w.p,
-                               (float *)c->act_s.p, u ? u + xo : nullptr, h ? h + xo : nullptr);
+            hipLaunchKernelGGL((k_act_q_tiles<256>), dim3(pb), dim3(256), 0, c->stream, x_dev + xo, mc, K, L.cb32, split, am,
+                               xt, as, u ? u + xo : nullptr, h ? h + xo : nullptr);
         else
-            hipLaunchKernelGGL((k_act_q_tiles<64>), dim3(pb), dim3(256), 0, c->stream, x_dev + xo, mc, K, L.cb32, split, am, (uint8_t *)c->act_w.p,
-                               (float *)c->act_s.p, u ? u + xo : nullptr, h ? h + xo : nullptr);
+            hipLaunchKernelGGL((k_act_q_tiles<64>), dim3(pb), dim3(256), 0, c->stream, x_dev + xo, mc, K, L.cb32, split, am,
+                               xt, as, u ? u + xo : nullptr, h ? h + xo : nullptr);
         prof_end(c, tok);
         HIPCHK(hipGetLastError());
         int blocks = 0;

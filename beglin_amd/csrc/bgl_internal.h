@@ -83,8 +83,9 @@ bgl_tensor *tensor_from_parts(const BglDevTensor &T, void *w, void *s0, void *s1
 int prof_begin(bgl_ctx *c, int phase);
 void prof_end(bgl_ctx *c, int token);
 int dbuf_reserve(bgl_ctx *c, DevBuf &b, size_t bytes, bool zero);
-// The same for act_w / act_s / act_sum, whose prepared operands (prep_reuse) are copied along.
-int dbuf_grow_kept(bgl_ctx *c, DevBuf &b, size_t bytes);
+// act_w / act_s / act_sum for the same call at fewer columns, which a caller may capture after this one
+// (nothing inside a capture); prepared operands in them (prep_reuse) are copied along.
+int act_reserve_fewer(bgl_ctx *c, size_t w, size_t s, size_t sum);
 // Bytes of per-call scratch the context holds; with release, frees it (the caller synchronizes).
 size_t ctx_scratch(bgl_ctx *c, bool release);
 int check_wt(int kind, int bits, int out, int in);

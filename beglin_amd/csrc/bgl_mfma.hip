@@ -672,18 +672,13 @@ static int mf_reserve_fewer(bgl_ctx *c, int n, const BglDevTensor *Ts, int M) {
     }
     const size_t pb = (size_t)fl * 4;
     const bool dig = !gemv_x_fuses(c, Ts[0].K) || Ts[0].K > BGL_GEMV_X_FUSE_MAX_K;
-    const struct { DevBuf *b; size_t bytes; } need[3] = {{&c->act_w, 2 * ng * 192}, {&c->act_s, 2 * ng * 4}, {&c->act_sum, 4 * ng * 16}};
-    bool have = c->part.bytes >= pb;
-    for (auto &d : need) have = have && (!dig || d.b->bytes >= d.bytes);
-    if (have) return 0;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    HIPCHK(hipStreamIsCapturing(c->stream, &cs));
-    if (cs != hipStreamCaptureStatusNone) return 0;                // this call may still have all that it needs
-    if (dbuf_reserve(c, c->part, pb, false)) return bgl_last_code();
-    if (dig)
-        for (auto &d : need)
-            if (dbuf_grow_kept(c, *d.b, d.bytes)) return bgl_last_code();
-    return 0;
+    if (c->part.bytes < pb) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        HIPCHK(hipStreamIsCapturing(c->stream, &cs));
+        if (cs != hipStreamCaptureStatusNone) return 0;            // this call may still have all that it needs
+        if (dbuf_reserve(c, c->part, pb, false)) return bgl_last_code();
+    }
+    return dig ? act_reserve_fewer(c, 2 * ng * 192, 2 * ng * 4, 4 * ng * 16) : 0;
 }
 
 // From 2 columns.  The dot4 kernels multiply three digits per value and column (k_gemv: 4 or 8 columns

@@ -140,3 +140,27 @@ def test_gemm_q_mlp_block(ctx, torch_dev, oracle, kind, M):
     assert np.array_equal(y.cpu().numpy().view(np.uint32), ref.view(np.uint32))
     for t in ts:
         t.free()
+
+
+@pytest.mark.parametrize("kind,rows,inn,M", [(1, 100, 256, 20), (2, 16400, 256, 6), (3, 70, 512, 64)])
+def test_gemm_q_leaves_prepared_operands(torch_dev, oracle, kind, rows, inn, M):
+    """A W4A8 call over a short K took no prepared operands of its own, so what bgl_prep_act_dev left
+    outlived it: k_gemm_q's codes lie elsewhere."""
+    import beglin_amd
+    say("gemm_q beside prepared operands", kind, rows, inn, M)
+    c = beglin_amd.Context(0)
+    packed = pack(oracle, kind, seeded_normal(800 + M, (rows, inn), 0.02))
+    pp, ps = oracle.quantize_q4g64(seeded_normal(801, (90, 1024), 0.02))
+    tp = c.bind(1, pp, ps, 90, 1024)
+    x, xp = columns(802, M, inn), seeded_normal(803, (3, 1024))
+    xpd, yp = torch_dev.from_numpy(xp).cuda(), torch_dev.empty((3, 90), device="cuda")
+    for act in (0, 1):
+        torch_dev.cuda.synchronize()
+        c.prep_only(xpd, act, tp)
+        run(c, torch_dev, kind, [packed], x, [None], [rows], [oracle.matmul_sdot(kind, packed[0], packed[1], x, sub=packed[2])])
+        c.matmul_prepped(tp, yp, act=act, M=3)
+        c.sync()
+        ref = oracle.matmul_sdot(1, pp, ps, xp) if act else oracle.gemm_f32(1, pp, ps, xp)
+        assert np.max(np.abs(yp.cpu().numpy() - ref)) <= 1e-5 * np.max(np.abs(ref))
+    tp.free()
+    c.close()
