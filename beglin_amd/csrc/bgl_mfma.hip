@@ -7,6 +7,12 @@
 // toward zero (x' - hi is exact in fp32): hi + lo holds x' to about 2^-21 of the column maximum.  v_mfma_f32_16x16x32_f16 multiplies exactly and
 // accumulates in fp32; each quantization group's partial sum is folded with its fp32 scale (one
 // FMA per output per group) and the column factor 2^-(14-e) is applied at the end.
+// The fp16 parts end at 2^-24, 2^-38 of the column's maximum over the split.  At 2..15 columns, which the
+// exact digits of the dot4 kernels held to 2^-23 of each 64-group's own maximum (2^-46 in groups of many
+// small elements), a column with such a group below 2^-14 of its maximum is multiplied a second time by
+// what the parts leave over (mf_wide, mf_leftover), so it is held to 2^-60.  (One test and the branch:
+// 28672 x 4096 at 5 columns 23.7 -> 24.0 us, 4096 x 4096 11.1 -> 11.4; a call with such a column takes
+// up to twice as long.)
 //
 // Layout.  A (weights, 16 rows x 32 k per instruction): lane l holds row l%16 and the 8 elements
 // 8*(l/16)..+7 of the 32-element K-step -- with the device's 16-byte chunk layout that is one
@@ -76,6 +82,7 @@ struct MfmaLaunch {
     int ntasks;
     int M;                   // valid columns (<= 16*CT)
     const float *x;          // activations x[m][k], M rows of K floats
+    int residual;            // columns of a wide range get a second product (one column tile only)
 };
 
 // ==================================================================================== GEMM kernel
@@ -120,6 +127,54 @@ __device__ __forceinline__ float mf_nonfinite(const BglDevTensor &T, int n, cons
     return acc;
 }
 
+// What the two fp16 parts of x * 2^sh leave over (exact; below 2^-8, as x * 2^sh is below 2^14): scaled by
+// 2^MF_RES_BITS, a second product's column.
+#define MF_RES_BITS 22
+__device__ __forceinline__ float mf_leftover(float x, int sh) {
+    const float v = ldexpf(x, sh);
+    const mf_h2 h = __builtin_bit_cast(mf_h2, __builtin_amdgcn_cvt_pkrtz(v, 0.0f));
+    const float r = v - (float)h[0];
+    const mf_h2 l = __builtin_bit_cast(mf_h2, __builtin_amdgcn_cvt_pkrtz(r, 0.0f));
+    return r - (float)l[0];
+}
+
+// Whether a wave's column (its slots in v, of which those below n are real; lo: the lane's smallest |x| bits,
+// e: the exponent of the column's largest magnitude) has a 64-value group with as many small elements as
+// bgl_x_level1 asks for, small being below 2^(e-14).  In the other groups at most 21 elements lie that low
+// and at least as many above, so the digits, 2^-23 of their largest, were no finer than the fp16 parts.
+template <int SPL>
+__device__ __forceinline__ bool mf_wide(const float4 (&v)[SPL][2], uint32_t lo, int n, int e) {
+    const float thr = ldexpf(1.0f, e - 14);
+    if (!__any(__uint_as_float(lo) < thr)) return false;
+    const int lane = threadIdx.x & 63;
+    bool wide = false;
+#pragma unroll
+    for (int j = 0; j < SPL; j++) {
+        const bool in = lane + 64 * j < n;
+        auto below = [&](float x) { return in && fabsf(x) < thr; };
+        int cnt = 0;                                               // over the wave's 8 groups, zeros too
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const float4 q = v[j][h];
+            cnt += __popcll(__ballot(below(q.x))) + __popcll(__ballot(below(q.y))) + __popcll(__ballot(below(q.z))) +
+                   __popcll(__ballot(below(q.w)));
+        }
+        if (cnt < BGL_X_SMALL_MAX) continue;                       // (more small than large is 33 of 64, zeros among them)
+        int c = 0;                                                 // small + 256 * large of the lane's 8, then of its group's 64
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const float4 q = v[j][h];
+            auto one = [&](float x) { return fabsf(x) >= thr ? 256 : x != 0.0f ? 1 : 0; };
+            c += one(q.x) + one(q.y) + one(q.z) + one(q.w);
+        }
+        c += dpp_i<0xB1>(c);
+        c += dpp_i<0x4E>(c);
+        c += dpp_i<0x141>(c);
+        wide = wide || (in && bgl_x_level1(c & 255, c >> 8));
+    }
+    return __any(wide);
+}
+
 template <int FMT, int NB, int CT, int KW>
 __global__ __launch_bounds__(MF_WAVES * KW * 64) void k_gemm_mfma(MfmaLaunch L) {
     constexpr int NT = MF_WAVES * KW * 64;
@@ -139,11 +194,18 @@ __global__ __launch_bounds__(MF_WAVES * KW * 64) void k_gemm_mfma(MfmaLaunch L) 
     __shared__ uint4 xs[KPM * XS];                                 // [step][CT][hi/lo][64 lanes], rows XS apart
     __shared__ uint4 ss[MF_TILES * UMAX * SUT];                    // [tile][unit][64 rows] scale words
 
+    __shared__ int cex[16 * MF_MAXCT];                             // per column: the exponent of its sums,
+    __shared__ int cnf[16 * MF_MAXCT];                             // whether it holds NaN or +-Inf in the split,
+    __shared__ int cwd[CT == 1 ? 16 : 1];                          // whether its range is wide (one column tile)
+    int level = 0;
+second_product:                                                    // level 1: added to what level 0 stored
+    int tid = threadIdx.x;
+    if constexpr (CT == 1) asm("" : "+v"(tid));                    // (opaque: no address kept in registers for it)
     const int ti = mf_task(L);
     const MfmaTask &tk = L.t[ti];
     const BglDevTensor &T = tk.T;
     // the wave index is uniform: in a scalar register, every offset derived from it is scalar too
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, q = lane >> 4;
     const int kw = wave / MF_WAVES, w8 = wave % MF_WAVES;          // K-slice, wave within the slice
     const int wt = w8 / (4 / MF_RBW), rbase = (w8 % (4 / MF_RBW)) * MF_RBW;   // tile in the group, first row block
     const int local = (int)blockIdx.x - tk.wg0;
@@ -202,9 +264,9 @@ __global__ __launch_bounds__(MF_WAVES * KW * 64) void k_gemm_mfma(MfmaLaunch L) 
         ss[(st * UMAX + uu) * SUT + rem % SUT] = uu * SPU < ns ? make_uint4(g[0], g[1], g[2], g[3]) : make_uint4(0, 0, 0, 0);
     };
     mf_u4 sreg;
-    if constexpr (EARLY) sreg = scale_ld((int)threadIdx.x);
+    if constexpr (EARLY) sreg = scale_ld(tid);
     else
-        for (int e = threadIdx.x; e < MF_TILES * nsu; e += NT) scale_st(e, scale_ld(e));
+        for (int e = tid; e < MF_TILES * nsu; e += NT) scale_st(e, scale_ld(e));
 
     // ---- the weight ring: local K-step s lives in slot (s - ls0) % D until it is computed ----
     const int tile_c = min(tile, T.ntiles - 1);                    // waves past the tensor read a real tile
@@ -227,8 +289,8 @@ __global__ __launch_bounds__(MF_WAVES * KW * 64) void k_gemm_mfma(MfmaLaunch L) 
     // Non-finite values (NaN, +-Inf) enter the fragments as 0 and flag the column; the store adds
     // their products code * scale * x one element at a time (IEEE propagation, as the reference's
     // fp32-product sums).
-    __shared__ int cex[16 * MF_MAXCT];
-    __shared__ int cnf[16 * MF_MAXCT];
+    int xe[CPW];                                                   // one column tile: the columns' exponents, and the
+    uint32_t xlo[CPW];                                             // lane's smallest |x| bits, for what follows the barrier
 #pragma unroll
     for (int ci = 0; ci < CPW; ci++) {
         const int m = ci * NW + wave;
@@ -236,14 +298,18 @@ __global__ __launch_bounds__(MF_WAVES * KW * 64) void k_gemm_mfma(MfmaLaunch L) 
         // the column's largest |x| bits over the split; Inf / NaN bits exceed every finite value's, so
         // only then (rare) are they zeroed and the maximum taken again
         uint32_t mb = 0u;
+        if constexpr (CT == 1) xlo[ci] = 0x7fffffffu;
 #pragma unroll
         for (int j = 0; j < SPL; j++)
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 const float4 v = xv[ci][j][h];
-                const uint32_t t = max(max(__float_as_uint(v.x) & 0x7fffffffu, __float_as_uint(v.y) & 0x7fffffffu),
-                                       max(__float_as_uint(v.z) & 0x7fffffffu, __float_as_uint(v.w) & 0x7fffffffu));
+                const uint32_t a = __float_as_uint(v.x) & 0x7fffffffu, b = __float_as_uint(v.y) & 0x7fffffffu;
+                const uint32_t c = __float_as_uint(v.z) & 0x7fffffffu, d = __float_as_uint(v.w) & 0x7fffffffu;
+                const uint32_t t = max(max(a, b), max(c, d));
                 mb = m < L.M && lane + 64 * j < 4 * ns ? max(mb, t) : mb;
+                // (slots past the split are copies of the column's first)
+                if constexpr (CT == 1) xlo[ci] = min(min(min(a, b), min(c, d)), xlo[ci]);
             }
         mb = wave_max_u32(mb);
         if (lane == 0) cnf[m] = 0;
@@ -264,21 +330,37 @@ __global__ __launch_bounds__(MF_WAVES * KW * 64) void k_gemm_mfma(MfmaLaunch L) 
                     screen(v.x); screen(v.y); screen(v.z); screen(v.w);
                 }
             mb = wave_max_u32(mb);
-            if (lane == 0) cnf[m] = 1;
+            if (lane == 0) cnf[m] = level ? 0 : 1;                 // (their products are added once)
         }
         const float mx = __uint_as_float(mb);
         int e = 0;
         if (mx > 0.0f) frexpf(mx, &e);                             // mx in [2^(e-1), 2^e)
         // x' = x * 2^(14-e), applied to each value (the factor alone leaves fp32's range for
         // e < -113, columns whose largest |x| is below 2^-114); the sums are unscaled by 2^(e-14)
-        const int sh = mx > 0.0f ? 14 - e : 0;
+        int sh = mx > 0.0f ? 14 - e : 0;
         if (lane == 0) cex[m] = -sh;
+        bool use = m < L.M;
+        if constexpr (CT == 1) {
+            if (level) {                                           // the split's leftover in place of the column
+#pragma unroll
+                for (int j = 0; j < SPL; j++)
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        float4 &v = xv[ci][j][h];
+                        v = make_float4(mf_leftover(v.x, sh), mf_leftover(v.y, sh), mf_leftover(v.z, sh), mf_leftover(v.w, sh));
+                    }
+                if (lane == 0) cex[m] = -sh - MF_RES_BITS;
+                sh = MF_RES_BITS;
+                use = use && cwd[m];                               // (this wave wrote it)
+            }
+            xe[ci] = e;
+        }
         const int ct = m >> 4, ml = m & 15;
 #pragma unroll
         for (int j = 0; j < SPL; j++) {
             const int g = lane + 64 * j;
             if (g >= 4 * nsr) break;
-            const bool ok = m < L.M && g < 4 * ns;
+            const bool ok = (CT == 1 ? use : m < L.M) && g < 4 * ns;
             const float4 a = xv[ci][j][0], b = xv[ci][j][1];
             const float v8[8] = {a.x, a.z, a.y, a.w, b.x, b.z, b.y, b.w};   // element order {0,2,1,3,4,6,5,7}
             // hi = fp16(x') rounded toward zero, two at a time; x' - hi is exact in fp32 (hi is x'
@@ -303,8 +385,18 @@ __global__ __launch_bounds__(MF_WAVES * KW * 64) void k_gemm_mfma(MfmaLaunch L) 
     }
     // the scales, into LDS (scale units past the split are zeroed)
     if constexpr (EARLY)
-        if ((int)threadIdx.x < MF_TILES * nsu) scale_st((int)threadIdx.x, sreg);
+        if (tid < MF_TILES * nsu) scale_st(tid, sreg);
     __syncthreads();
+    // (after the barrier, while the weights are on their way: nothing waits for it before the end)
+    if constexpr (CT == 1)
+        if (L.residual && !level) {
+#pragma unroll
+            for (int ci = 0; ci < CPW; ci++) {
+                const int m = ci * NW + wave;
+                const bool wide = m < L.M && mf_wide<SPL>(xv[ci], xlo[ci], 4 * ns, xe[ci]);
+                if (lane == 0) cwd[m] = wide;
+            }
+        }
 
     mf_f4 acc[MF_RBW][CT];
 #pragma unroll
@@ -441,7 +533,19 @@ __global__ __launch_bounds__(MF_WAVES * KW * 64) void k_gemm_mfma(MfmaLaunch L) 
 
     const int S = (KS + tk.kps - 1) / tk.kps;
     const int nb = tile0 * BGL_TILE;                                // first row of the workgroup
-    for (int i = threadIdx.x; i < 16 * CT * (OBR / 4); i += NT) {
+    if constexpr (CT == 1)
+        if (level) {                                               // onto what this thread stored
+            for (int i = tid; i < 16 * (OBR / 4); i += NT) {
+                const int m = i / (OBR / 4), nl = (i % (OBR / 4)) * 4, n = nb + nl;
+                if (m >= L.M || !cwd[m]) continue;
+                const float *a = ob + m * OBR + (nl ^ ((m & 15) << 2));
+                float *dst = (S > 1 ? tk.part + ((size_t)split * L.M + m) * T.N : tk.y + (size_t)m * tk.ystride) + n;
+                for (int e = 0; e < 4; e++)
+                    if (n + e < T.N) dst[e] += ldexpf(KW == 2 ? a[e] + a[16 * OBR + e] : a[e], cex[m]);
+            }
+            return;
+        }
+    for (int i = tid; i < 16 * CT * (OBR / 4); i += NT) {
         const int m = i / (OBR / 4), nl = (i % (OBR / 4)) * 4, n = nb + nl;
         if (m >= L.M || n >= T.N) continue;
         const int sw = nl ^ ((m & 15) << 2);
@@ -469,6 +573,17 @@ __global__ __launch_bounds__(MF_WAVES * KW * 64) void k_gemm_mfma(MfmaLaunch L) 
                 if (n + e < T.N) dst[e] = o[e];
         }
     }
+    if constexpr (CT == 1)
+        if (L.residual) {
+            int wide = 0;
+#pragma unroll
+            for (int m = 0; m < 16; m++) wide |= cwd[m];
+            if (wide) {                                            // uniform
+                level = 1;
+                __syncthreads();                                   // the stage is read out
+                goto second_product;
+            }
+        }
 }
 
 // ==================================================================================== K-split reduce
@@ -733,7 +848,7 @@ int run_gemm_mfma(bgl_ctx *c, int n, const BglDevTensor *Ts, const float *x_dev,
         const int CT = (Mc + 15) / 16;
         MfmaLaunch L;
         memset(&L, 0, sizeof L);
-        L.ntasks = n; L.M = Mc; L.x = x_dev + (size_t)m0 * K;
+        L.ntasks = n; L.M = Mc; L.residual = M < 16; L.x = x_dev + (size_t)m0 * K;
         int wgs = 0;
         size_t poff[BGL_MAX_TASKS], pfl = 0;              // partial offsets (floats) in the shared buffer
         int S_[BGL_MAX_TASKS];
