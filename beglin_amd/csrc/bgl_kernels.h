@@ -201,6 +201,7 @@ struct MoeTask {
     int ck;
     const void *xfr;             // k_moe_m: the rows' fp16 fragments and their {exponent, non-finite} pairs
     const int2 *xe;
+    size_t xres;                 //   from a row's fragments to those of its leftover, in 16 bytes
     int mbx;                     // k_moe_x: token columns of records the launch's LDS holds (4 or 8)
 };
 
@@ -256,5 +257,5 @@ int bgl_launch_moe_x2(const MoeTask &a, const MoeTask &b, int K, int nw, int cap
 bool bgl_moe_m_tensor(const BglDevTensor &T);
 size_t bgl_moe_frag_bytes(long rows, int K);
 void bgl_launch_moe_frag(const float *x0, int K0, int rows0, void *fr0, void *xe0, const float *x1, int K1, int rows1, void *fr1,
-                         void *xe1, hipStream_t st);
+                         void *xe1, size_t res, hipStream_t st);
 int bgl_launch_moe_m(const MoeTask &a, const MoeTask *b, hipStream_t st);

@@ -558,10 +558,15 @@ static int moe_digits_fewer(bgl_ctx *c, const bgl_tensor *const (&stacks)[3], co
     return 0;
 }
 
-// Bytes of the fragments and row exponents of a call, in one allocation with its fp32 rows (a context's
-// first call pays for each).
+// The scratch of a call behind its fp32 rows, in one allocation with them (a context's first call pays for
+// each): fragments of h, as much again for the rows' leftovers, then every row's exponent and flags.  Those
+// of x and their leftovers lie in the rows of the down projections, which come later, where those hold them.
+static bool moe_m_x_in_rows(int K, int Ish) { return K > 1 || Ish; }
+static size_t moe_m_frags(int T, int P, int H, int I, int Ish) {
+    return bgl_moe_frag_bytes(P, I) + bgl_moe_frag_bytes(T, Ish) + (moe_m_x_in_rows(P / T, Ish) ? 0 : bgl_moe_frag_bytes(T, H));
+}
 static size_t moe_m_bytes(int T, int P, int H, int I, int Ish) {
-    return bgl_moe_frag_bytes(T, H) + bgl_moe_frag_bytes(P, I) + bgl_moe_frag_bytes(T, Ish) + (size_t)(2 * T + P) * sizeof(int2);
+    return 2 * moe_m_frags(T, P, H, I, Ish) + (size_t)(2 * T + P) * sizeof(int2);
 }
 
 // The FFN's gathers through k_moe_m: fragments of x, gate+up (routed and shared in one launch),
@@ -570,10 +575,12 @@ static int moe_ffn_m(bgl_ctx *c, const bgl_tensor *gate, const bgl_tensor *up, c
                      const bgl_tensor *su, const bgl_tensor *sd, const float *x_dev, const MoeScratch &S, int T, int K, float *h,
                      float *shh, float *dd, float *sdd, uint8_t *fr) {
     const int H = gate->T.K, I = gate->T.N, Ish = sg ? sg->T.N : 0, P = T * K, E = (int)gate->experts.size();
-    uint8_t *xf = fr, *hf = xf + bgl_moe_frag_bytes(T, H), *sf = hf + bgl_moe_frag_bytes(P, I);
-    int2 *xe = (int2 *)(sf + bgl_moe_frag_bytes(T, Ish)), *he = xe + T, *se = he + P;
+    const bool xr = moe_m_x_in_rows(K, Ish);
+    uint8_t *hf = fr, *sf = hf + bgl_moe_frag_bytes(P, I), *xf = xr ? (uint8_t *)dd : sf + bgl_moe_frag_bytes(T, Ish);
+    const size_t res = moe_m_frags(T, P, H, I, Ish), xres = xr ? bgl_moe_frag_bytes(T, H) : res;
+    int2 *xe = (int2 *)(fr + 2 * res), *he = xe + T, *se = he + P;
     int tok = prof_begin(c, 0);
-    bgl_launch_moe_frag(x_dev, H, T, xf, xe, nullptr, H, 0, nullptr, nullptr, c->stream);
+    bgl_launch_moe_frag(x_dev, H, T, xf, xe, nullptr, H, 0, nullptr, nullptr, xres, c->stream);
     prof_end(c, tok);
     HIPCHK(hipGetLastError());
     MoeTask r, s;
@@ -583,11 +590,11 @@ static int moe_ffn_m(bgl_ctx *c, const bgl_tensor *gate, const bgl_tensor *up, c
     max_units(gate, r.tpe, units);
     r.ta = (const BglDevTensor *)gate->dev_table; r.tb = (const BglDevTensor *)up->dev_table;
     r.E = E; r.off = S.off; r.cols = S.tok; r.y = h; r.ystride = I; r.swiglu = 1;
-    r.xfr = xf; r.xe = xe; r.a.xf = x_dev;
+    r.xfr = xf; r.xe = xe; r.xres = xres / 16; r.a.xf = x_dev;
     if (sg) {
         s.da = sg->T; s.db = su->T; s.tpe = sg->T.ntiles; s.ncols = T; s.seg = 16; s.E = (T + 15) / 16;
         s.y = shh; s.ystride = Ish; s.swiglu = 1;
-        s.xfr = r.xfr; s.xe = r.xe; s.a.xf = x_dev;
+        s.xfr = r.xfr; s.xe = r.xe; s.xres = r.xres; s.a.xf = x_dev;
     }
     tok = prof_begin(c, 1);
     bgl_launch_moe_m(r, sg ? &s : nullptr, c->stream);
@@ -595,17 +602,17 @@ static int moe_ffn_m(bgl_ctx *c, const bgl_tensor *gate, const bgl_tensor *up, c
     HIPCHK(hipGetLastError());
     tok = prof_begin(c, 0);
     // (pairs whose expert id was out of range leave rows past the last segment unwritten; no segment reads them)
-    bgl_launch_moe_frag(h, I, P, hf, he, shh, Ish, sg ? T : 0, sf, se, c->stream);
+    bgl_launch_moe_frag(h, I, P, hf, he, shh, Ish, sg ? T : 0, sf, se, res, c->stream);
     prof_end(c, tok);
     HIPCHK(hipGetLastError());
     memset(&r, 0, sizeof r);
     max_units(down, r.tpe, units);
     r.ta = (const BglDevTensor *)down->dev_table; r.E = E; r.off = S.off; r.y = dd; r.ystride = H;
-    r.xfr = hf; r.xe = he; r.a.xf = h;
+    r.xfr = hf; r.xe = he; r.xres = res / 16; r.a.xf = h;
     if (sg) {
         memset(&s, 0, sizeof s);
         s.da = sd->T; s.tpe = sd->T.ntiles; s.ncols = T; s.seg = 16; s.E = (T + 15) / 16; s.y = sdd; s.ystride = H;
-        s.xfr = sf; s.xe = se; s.a.xf = shh;
+        s.xfr = sf; s.xe = se; s.xres = res / 16; s.a.xf = shh;
     }
     tok = prof_begin(c, 1);
     bgl_launch_moe_m(r, sg ? &s : nullptr, c->stream);

@@ -4,8 +4,9 @@
 // k_moe_x digitises every token in every tile's workgroup and multiplies three digits per value and token
 // on the vector ALUs: at 64 tokens of the DeepSeek-V2-Lite layer that is what bounds it (gate+up 282 us,
 // down 195 us for 470 and 240 MB).  Here a call's rows are split once into fp16 hi + lo (k_moe_frag;
-// bgl_mfma.hip has the numerics: exact weights, activations to 2^-21 of themselves) and a workgroup
-// multiplies 16 tokens at a time:
+// bgl_mfma.hip has the numerics: exact weights, activations to 2^-21 of themselves or 2^-38 of the row's
+// maximum; rows of a wide range once more, with what that leaves over) and a workgroup multiplies 16 tokens at
+// a time:
 //
 //   workgroup = one 64-row tile of one expert (gate and up rows together), 4 waves = 2 row halves x 2 K
 //   slices.  A wave streams its 32 rows' weights straight from HBM (a pair of K-steps ahead, or two for
@@ -36,13 +37,27 @@
 // ------------------------------------------------------------------ activation fragments
 // One workgroup per row: x' = x * 2^(14-e) (e: exponent of the row's largest finite |x|) as hi = fp16(x')
 // and lo = fp16(x' - hi), toward zero, in [row][K/32][hi: 32 halves | lo: 32 halves], eight values as
-// {0,2,1,3,4,6,5,7}; xe[row] = {e - 14, whether the row holds NaN or +-Inf (as 0 here)}.
+// {0,2,1,3,4,6,5,7}; xe[row] = {e - 14, bit 0: the row holds NaN or +-Inf (as 0 here)}.
+// A row of a wide range (a 64-value group with as many elements below 2^(e-14) as bgl_x_level1 asks for: the
+// parts then hold less than exact digits under that group's own exponent would) also gets the parts of what
+// hi and lo leave over, times 2^MM_RES_BITS, res further on, and bit 1 in xe[row].y.
+#define MM_RES_BITS 22
 struct MoeFrag {
     const float *x[2];
     uint4 *fr[2];
     int2 *xe[2];
     int K[2], rows0;             // rows [0, rows0) belong to set 0
+    size_t res;                  // from a row's parts to its leftover's, in uint4
 };
+// hi + lo of the scaled pair v0, v1; the leftover (exact, below 2^-8) in v0, v1
+__device__ __forceinline__ void mm_parts2(float &v0, float &v1, uint32_t &h, uint32_t &l) {
+    const mf_h2 hh = __builtin_bit_cast(mf_h2, __builtin_amdgcn_cvt_pkrtz(v0, v1));
+    v0 -= (float)hh[0]; v1 -= (float)hh[1];
+    const mf_h2 ll = __builtin_bit_cast(mf_h2, __builtin_amdgcn_cvt_pkrtz(v0, v1));
+    v0 -= (float)ll[0]; v1 -= (float)ll[1];
+    h = __builtin_bit_cast(uint32_t, hh);
+    l = __builtin_bit_cast(uint32_t, ll);
+}
 
 __global__ __launch_bounds__(256) void k_moe_frag(MoeFrag F) {
     __shared__ uint32_t red[4];
@@ -50,7 +65,7 @@ __global__ __launch_bounds__(256) void k_moe_frag(MoeFrag F) {
     const float *x = F.x[st] + (size_t)row * K;
     typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
     const int n8 = K / 8;
-    uint32_t mb = 0u, nf = 0u;
+    uint32_t mb = 0u, nf = 0u, lo = 0x7fffffffu;
     f4u a[2], c[2];                                       // the first two slots stay in registers
     for (int i = threadIdx.x, j = 0; i < n8; i += 256, j++) {
         const f4u v = *reinterpret_cast<const f4u *>(x + 8 * i), w = *reinterpret_cast<const f4u *>(x + 8 * i + 4);
@@ -61,6 +76,7 @@ __global__ __launch_bounds__(256) void k_moe_frag(MoeFrag F) {
             const uint32_t p = __float_as_uint(v[k]) & 0x7fffffffu, q = __float_as_uint(w[k]) & 0x7fffffffu;
             mb = max(mb, max(p < 0x7f800000u ? p : 0u, q < 0x7f800000u ? q : 0u));
             nf |= (p >= 0x7f800000u || q >= 0x7f800000u) ? 1u : 0u;
+            lo = min(lo, min(p, q));
         }
     }
     mb = wave_max_u32(mb);
@@ -74,22 +90,56 @@ __global__ __launch_bounds__(256) void k_moe_frag(MoeFrag F) {
     const float mx = __uint_as_float(mb);
     if (mx > 0.0f) frexpf(mx, &e);
     const int sh = mx > 0.0f ? 14 - e : 0;
-    if (threadIdx.x == 0) F.xe[st][row] = make_int2(-sh, (int)nf);
     uint4 *fr = F.fr[st] + (size_t)row * n8 * 2;
-    for (int i = threadIdx.x, j = 0; i < n8; i += 256, j++) {
+    auto slot = [&](int i, int j, float (&v8)[8]) {       // in the parts' order
         f4u v, w;
         if (j < 2) { v = j ? a[1] : a[0]; w = j ? c[1] : c[0]; }
         else { v = *reinterpret_cast<const f4u *>(x + 8 * i); w = *reinterpret_cast<const f4u *>(x + 8 * i + 4); }
-        const float v8[8] = {v.x, v.z, v.y, v.w, w.x, w.z, w.y, w.w};
+        const float t[8] = {v.x, v.z, v.y, v.w, w.x, w.z, w.y, w.w};
+#pragma unroll
+        for (int k = 0; k < 8; k++) v8[k] = isfinite(t[k]) ? t[k] : 0.0f;
+    };
+    for (int i = threadIdx.x, j = 0; i < n8; i += 256, j++) {
+        float v8[8];
+        slot(i, j, v8);
         uint32_t H[4], Lo[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            float v0 = v8[2 * k], v1 = v8[2 * k + 1];
-            v0 = isfinite(v0) ? ldexpf(v0, sh) : 0.0f;
-            v1 = isfinite(v1) ? ldexpf(v1, sh) : 0.0f;
-            const mf_h2 hh = __builtin_bit_cast(mf_h2, __builtin_amdgcn_cvt_pkrtz(v0, v1));
-            H[k] = __builtin_bit_cast(uint32_t, hh);
-            Lo[k] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(v0 - (float)hh[0], v1 - (float)hh[1]));
+            float v0 = ldexpf(v8[2 * k], sh), v1 = ldexpf(v8[2 * k + 1], sh);
+            mm_parts2(v0, v1, H[k], Lo[k]);
+        }
+        uint4 *d = fr + (i >> 2) * 8 + (i & 3);
+        d[0] = make_uint4(H[0], H[1], H[2], H[3]);
+        d[4] = make_uint4(Lo[0], Lo[1], Lo[2], Lo[3]);
+    }
+    bool wide = false;
+    const float thr = ldexpf(1.0f, e - 14);
+    if (__any(__uint_as_float(lo) < thr))                 // (a group's 8 slots are 8 lanes, all of them or none in the row)
+        for (int i = threadIdx.x, j = 0; i < n8; i += 256, j++) {
+            float v8[8];
+            slot(i, j, v8);
+            int n = 0;                                    // small + 256 * large
+#pragma unroll
+            for (int k = 0; k < 8; k++) n += fabsf(v8[k]) >= thr ? 256 : v8[k] != 0.0f ? 1 : 0;
+            n += dpp_i<0xB1>(n);
+            n += dpp_i<0x4E>(n);
+            n += dpp_i<0x141>(n);
+            wide = wide || bgl_x_level1(n & 255, n >> 8);
+        }
+    wide = __syncthreads_or(wide);
+    if (threadIdx.x == 0) F.xe[st][row] = make_int2(-sh, (int)(nf | (wide ? 2u : 0u)));
+    if (!wide) return;
+    fr += F.res;
+    for (int i = threadIdx.x, j = 0; i < n8; i += 256, j++) {
+        float v8[8];
+        slot(i, j, v8);
+        uint32_t H[4], Lo[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            float v0 = ldexpf(v8[2 * k], sh), v1 = ldexpf(v8[2 * k + 1], sh);
+            mm_parts2(v0, v1, H[k], Lo[k]);
+            v0 = ldexpf(v0, MM_RES_BITS); v1 = ldexpf(v1, MM_RES_BITS);
+            mm_parts2(v0, v1, H[k], Lo[k]);
         }
         uint4 *d = fr + (i >> 2) * 8 + (i & 3);
         d[0] = make_uint4(H[0], H[1], H[2], H[3]);
@@ -169,6 +219,7 @@ template <int FMT, int NB, bool GLU>
 __device__ __forceinline__ void moe_m_tile(const MoeTask &Mt, const BglDevTensor &Ta, const BglDevTensor &Tb, int tile, int s0, int s1,
                                            float *red) {
     constexpr int NM = GLU ? 2 : 1, PARTS = mm_parts<FMT, NB>();
+    constexpr int RES = MM_KS * NM * 1024;                        // red: the sums, then those of the leftover
     constexpr int RD = Planes<FMT, NB>::WORDS <= 4 ? 2 : 1;       // K-step pairs of weights in flight
     constexpr bool PERSTEP = FMT == BGL_Q4G32H || FMT == BGL_MXFP4;   // a scale per K-step (32 values), else per pair
     constexpr bool AFF = FMT == BGL_Q4G64A;
@@ -188,11 +239,11 @@ __device__ __forceinline__ void moe_m_tile(const MoeTask &Mt, const BglDevTensor
     const uint32_t tchunk = (uint32_t)tile * Ta.cpr;
     const uint32_t row4 = (32u * rh + (lane & 15)) * 4u;          // scale byte offset of row block 0's row
 
-    for (int c0 = s0; c0 < s1; c0 += MM_COLS) {
+    for (int c0 = s0, level = 0; c0 < s1;) {                      // level 1: rows of a wide range once more, with their leftover's parts
         // the lane's token (A operand row lane % 16; past the segment: its last one, not stored)
         const int sp = min(c0 + (lane & 15), s1 - 1);
         const int xrow = Mt.cols ? Mt.cols[sp] : sp;
-        const BGL_GLOBAL bgl_u32x4 *xp = (const BGL_GLOBAL bgl_u32x4 *)(Mt.xfr) + (size_t)xrow * (K >> 2) + q;
+        const BGL_GLOBAL bgl_u32x4 *xp = (const BGL_GLOBAL bgl_u32x4 *)(Mt.xfr) + (size_t)xrow * (K >> 2) + q + (level ? Mt.xres : 0);
         struct XF { mf_h8 h[2], l[2]; };
         auto load_x = [&](XF &f, int p) {
             const int pc = min(p, NP - 1);
@@ -278,8 +329,11 @@ __device__ __forceinline__ void moe_m_tile(const MoeTask &Mt, const BglDevTensor
         }
         if (p < p1) step(ring[0], xf[0], xf[1], p);
 
-        // the slices' sums through LDS: [slice][matrix][row half][row block][v][lane]
-        float *my = red + (size_t)ks * (NM * 1024) + rh * 512 + lane;
+        // the slices' sums through LDS: [slice][matrix][row half][row block][v][lane]; the tokens' exponents
+        // and flags (lane % 16) on their way meanwhile
+        const int sq = min(c0 + (lane & 15), s1 - 1), xr = Mt.cols ? Mt.cols[sq] : sq;
+        const int2 xq = Mt.xe[xr];
+        float *my = red + (level ? RES : 0) + (size_t)ks * (NM * 1024) + rh * 512 + lane;
 #pragma unroll
         for (int m = 0; m < NM; m++)
 #pragma unroll
@@ -287,20 +341,30 @@ __device__ __forceinline__ void moe_m_tile(const MoeTask &Mt, const BglDevTensor
 #pragma unroll
                 for (int v = 0; v < 4; v++) my[m * 1024 + b * 256 + v * 64] = acc[m][b][v];
         __syncthreads();
+        if (!level && __any(xq.y & 2)) {                          // uniform over the workgroup: the same 16 tokens
+            level = 1;
+            continue;
+        }
         for (int o = threadIdx.x; o < 1024; o += MM_WAVES * 64) {
-            const int tk = o >> 6, r = o & 63, n = tile * BGL_TILE + r, s = c0 + tk;
+            const int tk = __builtin_amdgcn_readfirstlane(o >> 6), r = o & 63, n = tile * BGL_TILE + r, s = c0 + tk;
             if (s >= s1 || n >= Ta.N) continue;
             const float *src = red + (r >> 5) * 512 + ((r >> 4) & 1) * 256 + (tk & 3) * 64 + 16 * (tk >> 2) + (r & 15);
-            const int row = Mt.cols ? Mt.cols[s] : s;
-            const int2 xe = Mt.xe[row];
+            const int row = __builtin_amdgcn_readlane(xr, tk);
+            const int ex = __builtin_amdgcn_readlane(xq.x, tk), fl = __builtin_amdgcn_readlane(xq.y, tk);
             float val[NM];
 #pragma unroll
             for (int m = 0; m < NM; m++) {
                 float t = 0.0f;
 #pragma unroll
                 for (int k = 0; k < MM_KS; k++) t += src[(k * NM + m) * 1024];
-                t = ldexpf(t, xe.x);
-                if (xe.y) {                                       // NaN, +-Inf: their products one at a time
+                t = ldexpf(t, ex);
+                if (fl & 2) {
+                    float u = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < MM_KS; k++) u += src[RES + (k * NM + m) * 1024];
+                    t += ldexpf(u, ex - MM_RES_BITS);
+                }
+                if (fl & 1) {                                     // NaN, +-Inf: their products one at a time
                     const float *x = Mt.a.xf + (size_t)row * K;
 #pragma unroll 1
                     for (int k = 0; k < K; k++)
@@ -312,6 +376,8 @@ __device__ __forceinline__ void moe_m_tile(const MoeTask &Mt, const BglDevTensor
             Mt.y[(size_t)(Mt.ymap ? Mt.ymap[s] : s) * Mt.ystride + n] = out;
         }
         __syncthreads();
+        level = 0;
+        c0 += MM_COLS;
     }
 }
 
@@ -326,9 +392,11 @@ __device__ __forceinline__ BglDevTensor mm_tensor(const BglDevTensor *p) {
     return t;
 }
 
+// (down: 3 waves per SIMD at most, else the compiler gives up registers for a fourth: 4 tokens of the mixed
+// layer 30.5 -> 37.8 us)
 template <bool GLU>
-__global__ __launch_bounds__(MM_WAVES * 64, 3) void k_moe_m(MoePair P) {
-    __shared__ float red[MM_KS * (GLU ? 2 : 1) * 1024];
+__global__ __launch_bounds__(MM_WAVES * 64) __attribute__((amdgpu_waves_per_eu(3, GLU ? 8 : 3))) void k_moe_m(MoePair P) {
+    __shared__ float red[2 * MM_KS * (GLU ? 2 : 1) * 1024];
     const int second = (int)blockIdx.x >= P.nb0, b = second ? (int)blockIdx.x - P.nb0 : (int)blockIdx.x;
     MoeTask Mt = P.t[0];
     if (second) Mt = P.t[1];
@@ -378,17 +446,18 @@ bool bgl_moe_m_tensor(const BglDevTensor &T) {
 size_t bgl_moe_frag_bytes(long rows, int K) { return (size_t)rows * K * 4; }
 
 void bgl_launch_moe_frag(const float *x0, int K0, int rows0, void *fr0, void *xe0, const float *x1, int K1, int rows1, void *fr1,
-                         void *xe1, hipStream_t st) {
+                         void *xe1, size_t res, hipStream_t st) {
     MoeFrag F;
     F.x[0] = x0; F.x[1] = x1;
     F.fr[0] = (uint4 *)fr0; F.fr[1] = (uint4 *)fr1;
     F.xe[0] = (int2 *)xe0; F.xe[1] = (int2 *)xe1;
     F.K[0] = K0; F.K[1] = K1;
     F.rows0 = rows0;
+    F.res = res / 16;
     hipLaunchKernelGGL(k_moe_frag, dim3(rows0 + rows1), dim3(256), 0, st, F);
 }
 
-// The tasks' xfr / xe hold their rows' fragments; b null: one task.  Both are SwiGLU launches or neither.
+// The tasks' xfr / xe / xres hold their rows' fragments; b null: one task.  Both are SwiGLU launches or neither.
 int bgl_launch_moe_m(const MoeTask &a, const MoeTask *b, hipStream_t st) {
     if (b && a.swiglu != b->swiglu) return -1;
     MoePair P;

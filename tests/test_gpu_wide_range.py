@@ -1,13 +1,16 @@
 """Finite fp32 activations of a wide range, through the kernels that split them into fp16 parts at few
-columns (k_gemm_mfma at 2..15): channels of up to 1e8 whose weights are zero, so that the result comes
-from elements far below the largest one.  As exact digits (k_act_x24) such elements are held to 2^-46 of
-their 64-group's largest; the fp16 parts alone reach 2^-38 of a whole K split's largest, so columns of a
-wide range are multiplied a second time by what the first parts leave over.  Bar: max|y - ref| / max|ref| <= 1e-5 per column, as everywhere."""
+columns (k_gemm_mfma at 2..15, k_moe_frag + k_moe_m): channels of up to 1e8 whose weights are zero, so that
+the result comes from elements far below the largest one.  As exact digits (k_act_x24) such elements are
+held to 2^-46 of their 64-group's largest; the fp16 parts alone reach 2^-38 of a whole K split's or row's
+largest, so columns of a wide range are multiplied a second time by what the first parts leave over.  Bar: max|y - ref| / max|ref| <= 1e-5 per column, as everywhere."""
 import numpy as np
 import pytest
 
 from golden.fixtures import seeded_normal
-from test_gpu_outliers import TOL, check_classes, context, make_weights, relerr, run_dense, say, torch_dev  # noqa: F401
+from oracle_ffi import moe_ffn
+from test_gpu_moe import desc
+from test_gpu_moe import run_moe as run_layer
+from test_gpu_outliers import TOL, check_classes, context, make_weights, quant, relerr, run_dense, say, torch_dev  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
@@ -77,4 +80,78 @@ def test_few_columns_group(torch_dev, oracle, monkeypatch, K):  # noqa: F811
             check_classes(y[m].cpu().numpy(), ref[m], (K, m))
     for t in ts:
         t.free()
+    c.close()
+
+
+def layer(oracle, fmts, E, H, I, Ish, seed, wm_h, wm_i, up_rows=None):
+    """Experts (gate, up, down) and shared ones: columns by wm_h (gate, up) and wm_i (down); up's rows
+    by up_rows."""
+    def one(kind, bits, o, i, s, wm, rows):
+        w = seeded_normal(s, (o, i), 0.02) * wm[None, :].astype(np.float32)
+        if rows is not None:
+            w = w * rows[:, None]
+        w = np.ascontiguousarray(w, np.float32)
+        if kind == 6:                                  # int4 affine: codes 0..15 over each group's range
+            g = w.reshape(o, -1, 64)
+            b = g.min(-1)
+            s_ = (g.max(-1) - b) / np.float32(15)
+            q = np.rint((g - b[..., None]) / np.where(s_ > 0, s_, 1)[..., None]).astype(np.uint8).reshape(o, i)
+            return (6, 4, np.ascontiguousarray(q[:, ::2] | (q[:, 1::2] << 4)), s_.astype(np.float32), b.astype(np.float32))
+        if kind == 9:
+            return desc(oracle, 9, 4, w)
+        return (kind, bits, *quant(oracle, kind, w, bits))
+    pick = lambda e: fmts[e % len(fmts)]  # noqa: E731
+    gate = [one(*pick(e), I, H, seed + 3 * e, wm_h, None) for e in range(E)]
+    up = [one(*pick(e), I, H, seed + 3 * e + 1, wm_h, up_rows) for e in range(E)]
+    down = [one(*pick(e), H, I, seed + 3 * e + 2, wm_i, None) for e in range(E)]
+    if not Ish:
+        return gate, up, down, None
+    k = fmts[0] if fmts[0][0] not in (6, 9) else (1, 0)
+    sh = (one(*k, Ish, H, seed + 90, wm_h, None), one(*k, Ish, H, seed + 91, wm_h, None), one(*k, H, Ish, seed + 92, np.ones(Ish, np.float32), None))
+    return gate, up, down, sh
+
+
+@pytest.mark.parametrize("fmts", [[(1, 0)], [(5, 0), (2, 0)], [(4, 7), (4, 13)], [(6, 4)]])
+@pytest.mark.parametrize("T,Ish,K", [(3, 128, 3), (9, 0, 3), (40, 192, 3), (10, 0, 1)])
+def test_routed_rows(torch_dev, oracle, monkeypatch, fmts, T, Ish, K):  # noqa: F811
+    """Token rows of a wide range (x), beside ordinary ones.  Affine int4 has no zero columns: its large
+    channels fill whole groups, whose scale and bias are zero."""
+    c = context(monkeypatch)
+    E, H, I = 4, 320, 192
+    for i, name in enumerate(NAMES):
+        if fmts == [(6, 4)] and name != "half_1e6":
+            continue
+        say("wide routed rows", fmts, T, Ish, K, name)
+        x, wmul = wide(name, H, T, 920 + i)
+        if name == "half_1e6":
+            wmul[:] = 1.0; wmul[:128] = 0.0
+            x = seeded_normal(926, (T, H)); x[:, :128] *= np.float32(3e7)
+        x[T - 1] = seeded_normal(927 + i, (H,))
+        gate, up, down, sh = layer(oracle, fmts, E, H, I, Ish, 930 + 10 * i, wmul, np.ones(I, np.float32))
+        idx, w = oracle.route(seeded_normal(940 + i, (T, E)), K, True)
+        got = run_layer(c, torch_dev, gate, up, down, sh, x, idx, w)
+        ref = moe_ffn(oracle, gate, up, down, sh, H, I, x, idx, w)
+        for t in range(T):
+            assert relerr(got[t], ref[t]) <= TOL, (name, t, relerr(got[t], ref[t]))
+    c.close()
+
+
+@pytest.mark.parametrize("fmts", [[(1, 0)], [(2, 0), (4, 14)], [(4, 9), (4, 5)]])
+@pytest.mark.parametrize("T,Ish", [(4, 64), (12, 0)])
+def test_routed_inner_rows(torch_dev, oracle, monkeypatch, fmts, T, Ish):  # noqa: F811
+    """The same for h: every 64th value of the experts' up projection is 1e7 times the others, and the
+    down projection's column there is zero."""
+    c = context(monkeypatch)
+    E, H, I, K = 4, 192, 320, 3
+    say("wide inner rows", fmts, T, Ish)
+    rows, wmul = np.ones(I, np.float32), np.ones(I, np.float32)
+    rows[5::64] = 1e7
+    wmul[5::64] = 0.0
+    gate, up, down, sh = layer(oracle, fmts, E, H, I, Ish, 950, np.ones(H, np.float32), wmul, rows)
+    x = seeded_normal(960, (T, H))
+    idx, w = oracle.route(seeded_normal(961, (T, E)), K, True)
+    got = run_layer(c, torch_dev, gate, up, down, sh, x, idx, w)
+    ref = moe_ffn(oracle, gate, up, down, sh, H, I, x, idx, w)
+    for t in range(T):
+        assert relerr(got[t], ref[t]) <= TOL, (t, relerr(got[t], ref[t]))
     c.close()
