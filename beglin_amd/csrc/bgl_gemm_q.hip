@@ -380,6 +380,10 @@ static size_t gq_lds(int units) { return (size_t)(1 + (units + 3) / 4 * 4) * GQ_
 //   g256sf  28672 x 4096 41.8 / 21.0 (2: 26.7 / 20.6)         17920 x 1536 12.1 / 12.7 (16: 18.3 / 13.1)
 //           4096 x 14336 15.0 / 18.5
 //   q8g64   28672 x 4096 41.2 / 30.4 (4: 31.1 / 30.5)         17920 x 1536 26.5 / 12.1
+// More than 16 columns over few rows, 17 / 64 columns (the rows do not matter up to 3072: a wave walks K
+// alone): 64 rows q4g64 K = 512 8.4 / 7.3 and 22.7 / 7.6, 4096 16.0 / 11.4 and 39.0 / 12.2, 14336 53.4 / 25.1
+// and 172.7 / 29.1; g256sf 512 8.3 / 7.5 and 22.7 / 7.5, 14336 23.7 / 18.4 and 62.4 / 23.2; q8g64 512 7.9 / 7.5
+// and 21.3 / 7.6, 14336 49.7 / 23.7 and 161.1 / 26.9.
 bool gemm_q_ok(bgl_ctx *c, const BglDevTensor *Ts, int n, int M) {
     if (c->no_qmfma || M < 2) return false;
     const int fmt = Ts[0].fmt, K = Ts[0].K;

@@ -498,17 +498,19 @@ extern "C" int bgl_gather_matvec_dev(bgl_ctx *c, const bgl_tensor *experts, cons
 }
 
 // Whether a routed FFN of T tokens runs k_moe_m (bgl_moe_m.hip): every tensor in a format it takes, and
-// enough work for its two fragment launches and the combine.  Measured on the DeepSeek-V2-Lite layer (64
-// experts, top 6), us, k_moe_x or k_moe_gemv / k_moe_m:
-//   with shared experts (one launch with the routed ones)  mixed formats: 2 tokens 92.4 / 100.8, 3: 119.7 /
-//     116.8, 8: 178.7 / 167.3, 64: 540.5 / 273.1; int4: 1: 48.6 / 49.2, 3: 84.4 / 63.9; affine int4: 1: 56.5 /
-//     51.3, 64: 528 / 174
-//   without                                                mixed: 8: 130.0 / 150.8, 16: 184.3 / 196.2; int4 3:
-//     58.8 / 59.5, 12: 117.4 / 104.6; affine int4: 2: 46.2 / 55.0, 3: 73.4 / 65.6; 32 experts of 2880 x 2880, top 8,
-//     mixed: 4: 210 / 238, 8: 282.7 / 276.6, 14: 404 / 297
-// (two pairs per expert is where mixed formats break even; k_moe_m with 4 K slices, the 2 it has now are up
-// to 8% faster).  MXFP4 experts beside AF int4 ones stay refused,
-// and the tuning switches of k_moe_x keep it.
+// enough work for its two fragment launches and the combine.  Measured, us, k_moe_x or k_moe_gemv / k_moe_m,
+// means over six layers and inputs, DeepSeek-V2-Lite (64 experts, top 6) unless said:
+//   with shared experts (one launch with the routed ones)  mixed formats: 2 tokens 84.5 / 95.7, 3: 103.5 /
+//     101.6, 4: 129.9 / 110.5; int4: 1: 47.1 / 53.6, 2: 64.5 / 57.2, 3: 81.9 / 58.2; affine int4: 1: 56.6 / 57.0,
+//     2: 78.8 / 62.2; one layer at 128 and 512 tokens (shared experts read once per 16 tokens here, 64 in the
+//     dense block): mixed 951 / 304 and 3679 / 872, int4 660 / 202 and 2616 / 612
+//   without                                                mixed: 10: 144.1 / 145.4, 12: 158.6 / 157.0, 22: 215.2 /
+//     182.2; int4: 2: 46.8 / 53.4, 3: 55.8 / 54.2; affine int4: 2: 57.6 / 58.8, 3: 78.2 / 59.9; 32 experts of
+//     2880 x 2880, top 8, mixed: 4: 193 / 215, 8: 282 / 260; 8 experts of 4096 x 14336, top 2, int4: 1: 75 / 91,
+//     2: 158 / 129, 8: 347 / 203
+// So the line is where k_moe_m has not been seen to lose: two pairs per expert without shared experts (the
+// widest mixed layers break even there, int4 ones well before), else the counts below.  MXFP4 experts beside
+// AF int4 ones stay refused, and the tuning switches of k_moe_x keep it.
 // moe_m_below: the most tokens that stay with the other gathers (aff: an affine int4 tensor among them).
 static int moe_m_below(const bgl_tensor *const (&stacks)[3], const bgl_tensor *const (&shared)[3], bool aff, int K) {
     if (shared[0]) return aff ? 0 : 2;
