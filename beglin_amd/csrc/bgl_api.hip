@@ -933,10 +933,9 @@ static int run_gemv_q(bgl_ctx *c, int n, const BglDevTensor *Ts, const float *x_
         if (rc) return rc;
     }
     for (int m0 = 0; m0 < M;) {
-        const bool qml = qm && M - m0 >= QM_MIN_COLS;
-        const int mc = std::min(qml ? 16 : mbq, M - m0), MB = q_mb(mc);
+        const int mc = std::min(qm ? 16 : mbq, M - m0), MB = q_mb(mc);
         m0 += mc;
-        if (qml) {
+        if (qm) {                                            // all of them (more than 16 run k_gemm_q)
             GemvLaunch L;
             memset(&L, 0, sizeof L);
             int blocks = 0;
