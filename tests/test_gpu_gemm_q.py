@@ -68,7 +68,10 @@ def run(ctx, torch, kind, packed, x, biases, shapes, bits_equal_to):
 SHAPES = [(1, 77, 64, 17), (1, 200, 1024, 33), (1, 64, 4096, 65), (2, 130, 640, 48), (2, 50, 192, 130), (3, 65, 256, 64),
           (3, 100, 2304, 49), (10, 90, 1536, 31),
           (1, 16330, 192, 6), (3, 16400, 4096, 2), (3, 16400, 512, 9), (2, 90, 4160, 9),   # 2..16 columns
-          (1, 16330, 192, 40), (1, 8200, 576, 64), (2, 16330, 320, 17), (3, 16400, 768, 64)]
+          (1, 16330, 192, 40), (1, 8200, 576, 64), (2, 16330, 320, 17), (3, 16400, 768, 64),
+          # 32-row tiles in two launches (64 + 6 columns); a long K over few rows, its scales past 64 KB of
+          # LDS (from K = 16192 in groups of 64), to the longest K that the W4A8 kernels take (34880; 140 KB)
+          (1, 16400, 192, 70), (1, 70, 14336, 24), (1, 70, 16384, 33), (2, 40, 34880, 20), (3, 64, 49152, 17)]
 
 
 @pytest.mark.parametrize("kind,out,inn,M", SHAPES)
@@ -89,6 +92,34 @@ def test_gemm_q_group_with_biases(ctx, torch_dev, oracle):
     bias = [seeded_normal(60 + o, (o,), 1.0) if i != 1 else None for i, o in enumerate(outs)]
     ref = [oracle.matmul_sdot(1, p, s, x, bias=b) for (p, s, _), b in zip(packed, bias)]
     run(ctx, torch_dev, 1, packed, x, bias, outs, ref)
+
+
+@pytest.mark.parametrize("kind", [1, 2, 3])
+@pytest.mark.parametrize("out,inn,M", [(70, 512, 20), (70, 512, 70), (16400, 256, 20)])
+def test_gemm_q_nonfinite_columns(ctx, torch_dev, oracle, kind, out, inn, M):
+    """Columns with NaN or +-Inf (every code of the group 0 and its scale NaN or Inf, so every output row NaN),
+    with a group of zeros, and of values below 1e-8 (the floor of the scale); the finite columns bit for bit."""
+    say("gemm_q nonfinite", kind, out, inn, M)
+    pk, sc, sub = pack(oracle, kind, seeded_normal(820 + kind, (out, inn), 0.02))
+    x = seeded_normal(821 + M, (M, inn), 1.0)
+    x[1, 5], x[3, inn - 1], x[4, 70] = np.nan, np.inf, -np.inf
+    x[5, 7], x[5, 9] = np.inf, np.nan
+    x[7, :256], x[8, :256] = 0.0, x[8, :256] * np.float32(1e-10)
+    x[M - 1, 100] = np.nan
+    with np.errstate(all="ignore"):
+        ref = oracle.matmul_sdot(kind, pk, sc, x, sub=sub)
+    bad = [1, 3, 4, 5, M - 1]
+    assert np.isnan(ref[bad]).all() and np.isfinite(np.delete(ref, bad, 0)).all()
+    t = ctx.bind(kind, pk, sc, out, inn, sub=sub)
+    xd, y = torch_dev.from_numpy(x).cuda(), torch_dev.zeros((M, out), device="cuda")
+    torch_dev.cuda.synchronize()
+    ctx.matmul(t, xd, y, act=1)
+    ctx.sync()
+    got = y.cpu().numpy()
+    t.free()
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    ok = ~np.isnan(ref)
+    assert np.array_equal(got[ok].view(np.uint32), ref[ok].view(np.uint32))
 
 
 @pytest.mark.parametrize("kind,out", [(1, 70), (3, 70), (1, 16384)])

@@ -487,10 +487,10 @@ def test_w4a8_batched_prep_equals_fused(torch_dev, oracle, monkeypatch, kind):
 
 @pytest.mark.parametrize("kind,inn", [(1, 1536), (2, 1024), (3, 1536), (3, 8960), (1, 8960)])
 def test_w4a8_matrix_cores_equal_dot4(torch_dev, oracle, monkeypatch, kind, inn):
-    """W4A8 at 5..16 columns on the matrix cores (k_gemv_qm) against the dot4 kernel
-    (BGL_NO_QMFMA=1) and the oracle, bit for bit: column counts that fill one launch, leave a
-    partial one, and leave a 1-4 column remainder for the dot4 kernel (17, 21); a fused group of two
-    tensors with biases; columns quantized in the kernel and up front (BGL_Q_PREP=1)."""
+    """W4A8 at 5..16 columns on the matrix cores (k_gemv_qm; 17 and 21: k_gemm_q) against the dot4 kernel
+    (BGL_NO_QMFMA=1: launches of 8 and a remainder) and the oracle, bit for bit: column counts that fill one
+    launch and leave a partial one; a fused group of two tensors with biases; columns quantized in the
+    kernel and up front (BGL_Q_PREP=1)."""
     import beglin_amd
     torch = torch_dev
     outs_n = (200, 72)

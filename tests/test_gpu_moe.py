@@ -506,7 +506,8 @@ def test_moe_x_matches_prep_path(torch_dev, oracle, monkeypatch, T, tr):
     gate, up, down, shared = moe_setup(oracle, 6000 + T, E, H, I, Ish, fm, down_fmts=fm[::-1], sh_fmt=(4, 12))
     x = seeded_normal(90 + T, (T, H))
     idx, w = oracle.route(seeded_normal(91 + T, (T, E)), K, True)
-    outs = []
+    outs, preps = [], []
+    monkeypatch.setenv("BGL_NO_MFMA", "1")              # (more than two tokens run k_moe_m otherwise)
     for flag in ("0", "1"):
         monkeypatch.setenv("BGL_NO_MOE_X", flag)
         if tr:
@@ -514,8 +515,11 @@ def test_moe_x_matches_prep_path(torch_dev, oracle, monkeypatch, T, tr):
         else:
             monkeypatch.delenv("BGL_FORCE_TR", raising=False)
         c = beglin_amd.Context(0)
+        c.prof_enable()
         outs.append(run_moe(c, torch, gate, up, down, shared, x, idx, w))
+        preps.append(c.prof_read()["prep"][1])
         c.close()
+    assert preps[0] == 0 and preps[1] > 0               # the kernels that ran
     ref = moe_ffn(oracle, gate, up, down, shared, H, I, x, idx, w)
     assert relerr(outs[0], ref) <= TOL and relerr(outs[1], ref) <= TOL and relerr(outs[0], outs[1]) <= 2 * TOL
 
@@ -524,26 +528,38 @@ def test_moe_x_matches_prep_path(torch_dev, oracle, monkeypatch, T, tr):
 def test_moe_shared_on_matrix_cores(torch_dev, oracle, monkeypatch, T, sh_fmt):
     """From 16 tokens on, shared experts in a format the matrix cores decode exactly (int8, int4 g32,
     qNg64 n <= 10) run as a dense MLP block on the matrix cores (gate+up, SwiGLU, down) and the
-    combine adds their rows; n = 12 stays in the exact-digit gathers.  Both against the oracle's FFN
-    and against the gathers alone (BGL_NO_MFMA=1); hidden 320 (a partial pass of 256), shared width
+    combine adds their rows, where a dense routed expert keeps the call from k_moe_m; n = 12 stays in the
+    exact-digit gathers.  Without the dense expert the whole call runs k_moe_m.  All against the oracle's
+    FFN and against the gathers alone (BGL_NO_MFMA=1); hidden 320 (a partial pass of 256), shared width
     320, routed experts in mixed formats."""
     import beglin_amd
     torch = torch_dev
     E, H, I, K, Ish = 6, 320, 192, 2, 320
     say("moe shared matrix cores", T, sh_fmt)
-    fm = [(5, 0), (2, 0), (4, 7), (4, 15)]
-    gate, up, down, shared = moe_setup(oracle, 6300 + T, E, H, I, Ish, fm, down_fmts=fm[::-1], sh_fmt=sh_fmt)
-    x = seeded_normal(6310 + T, (T, H))
-    idx, w = oracle.route(seeded_normal(6320 + T, (T, E)), K, True)
-    outs = []
-    for flag in ("0", "1"):
-        monkeypatch.setenv("BGL_NO_MFMA", flag)
-        c = beglin_amd.Context(0)
-        outs.append(run_moe(c, torch, gate, up, down, shared, x, idx, w))
-        c.close()
-    monkeypatch.delenv("BGL_NO_MFMA", raising=False)
-    ref = moe_ffn(oracle, gate, up, down, shared, H, I, x, idx, w)
-    assert relerr(outs[0], ref) <= TOL and relerr(outs[1], ref) <= TOL and relerr(outs[0], outs[1]) <= 2 * TOL
+    for dense in (True, False):
+        fm = [(5, 0), (2, 0), (4, 7), (7, 16) if dense else (4, 15)]
+        gate, up, down, shared = moe_setup(oracle, 6300 + T, E, H, I, Ish, fm, down_fmts=fm[::-1], sh_fmt=sh_fmt)
+        x = seeded_normal(6310 + T, (T, H))
+        idx, w = oracle.route(seeded_normal(6320 + T, (T, E)), K, True)
+        outs, n = [], []
+        for flag in ("0", "1"):
+            monkeypatch.setenv("BGL_NO_MFMA", flag)
+            c = beglin_amd.Context(0)
+            c.prof_enable()
+            outs.append(run_moe(c, torch, gate, up, down, shared, x, idx, w))
+            p = c.prof_read()
+            n.append((p["prep"][1], p["gemv"][1], p["other"][1]))
+            c.close()
+        # launches (preparation, products, others): the bucketing and the combine, and the dense block's reduces
+        if not dense:
+            assert n[0] == (2, 2, 2), n                 # k_moe_frag and k_moe_m, twice
+        elif sh_fmt != (4, 12):
+            assert n[0][2] > n[1][2] or n[0][0] < n[1][0], n
+        else:
+            assert n[0] == n[1], n
+        monkeypatch.delenv("BGL_NO_MFMA", raising=False)
+        ref = moe_ffn(oracle, gate, up, down, shared, H, I, x, idx, w)
+        assert relerr(outs[0], ref) <= TOL and relerr(outs[1], ref) <= TOL and relerr(outs[0], outs[1]) <= 2 * TOL
 
 
 @pytest.mark.parametrize("T", [1, 3, 6, 13])
@@ -627,10 +643,14 @@ def test_mxfp4_decode_bitexact(ctx, torch_dev, oracle):
     t.free()
 
 
-@pytest.mark.parametrize("T", [1, 6, 21])
-def test_mxfp4_moe_ffn(ctx, torch_dev, oracle, T):
+@pytest.mark.parametrize("T,mfma", [(1, True), (6, True), (21, True), (6, False), (21, False)])
+def test_mxfp4_moe_ffn(torch_dev, oracle, monkeypatch, T, mfma):
     """The routed SwiGLU FFN with MXFP4 experts beside q4g32h and qNg64 ones (one gather launch
-    serves every format), shared experts in MXFP4, against the oracle's bucketed FFN."""
+    serves every format), shared experts in MXFP4, against the oracle's bucketed FFN: k_moe_x, and from
+    three tokens k_moe_m (mfma)."""
+    import beglin_amd
+    monkeypatch.setenv("BGL_NO_MFMA", "0" if mfma else "1")
+    ctx = beglin_amd.Context(0)
     torch = torch_dev
     say("mxfp4 moe ffn", T)
     E, H, I, K, Ish = 6, 320, 192, 2, 128

@@ -16,9 +16,9 @@ its column NaN; +-Inf gives +-Inf where every product with it has that sign, NaN
 an Inf channel is zero or products of both signs meet.  The tests compare the NaN / +Inf / -Inf
 pattern of every output with the oracle's, and the finite outputs to the 1e-5 bar.
 
-Kernels: k_gemv_x (M=1, digits made in the kernel and prepared), k_gemv (M = 4 / 8, and M = 32 with
-the matrix cores switched off), k_gemm_mfma (M = 32), k_moe_x and k_moe_gemv (routed MoE FFN at the
-DeepSeek-V2-Lite expert shape).  Bar: max|y - ref| / max|ref| <= 1e-5."""
+Kernels: k_gemv_x (M=1, digits made in the kernel and prepared), k_gemv (M = 4 / 8 / 32 with the matrix
+cores switched off), k_gemm_mfma (M = 4 / 8 / 32), k_moe_x and k_moe_gemv (routed MoE FFN at the
+DeepSeek-V2-Lite expert shape; several tokens with the matrix cores switched off), k_moe_m (several tokens).  Bar: max|y - ref| / max|ref| <= 1e-5."""
 import sys
 
 import numpy as np
@@ -163,19 +163,21 @@ MAJ_DENSE = [(5, 0, 8960, 1536), (4, 2, 14336, 4096), (4, 15, 14336, 4096), (4, 
 @pytest.mark.parametrize("kind,bits,N,K", MAJ_DENSE)
 def test_dense_majority_outliers(torch_dev, oracle, monkeypatch, kind, bits, N, K):
     """33 or 40 of every group's 64 channels at x1e2 .. x1e4 with zero weight columns: k_gemv_x
-    (digits made in the kernel, and by the prep kernel) at M = 1, k_gemv at M = 4 and the matrix
-    cores (or, for qNg64 n > 10, k_gemv) at M = 32 on the first 2048 rows, all to the 1e-5 bar.
+    (digits made in the kernel, and by the prep kernel) at M = 1, k_gemv and the matrix cores at M = 4 and
+    the matrix cores (or, for qNg64 n > 10, k_gemv) at M = 32 on the first 2048 rows, all to the 1e-5 bar.
     The weights of a pattern are quantized once and serve every configuration."""
     torch = torch_dev
-    ctxs = {"fused": context(monkeypatch), "prep": context(monkeypatch, BGL_X_FUSE=0)}
+    ctxs = {"fused": context(monkeypatch), "prep": context(monkeypatch, BGL_X_FUSE=0), "dot4": context(monkeypatch, BGL_NO_MFMA=1)}
     monkeypatch.delenv("BGL_X_FUSE", raising=False)
+    monkeypatch.delenv("BGL_NO_MFMA", raising=False)
     NR = min(N, 2048)                                   # rows of the 32-column run
     for i, pat in enumerate(MAJORITY):
         x, wmul = outlier_case(pat, K, 32, 800 + i)
         pk, sc = make_weights(oracle, kind, bits, N, K, wmul, 820 + i)
         ref14 = oracle.gemm_f32(kind, pk, sc, x[:4], bits=bits)
         ref32 = oracle.gemm_f32(kind, pk[:NR], sc[:NR], x, bits=bits)
-        for name, c, M in (("fused", ctxs["fused"], 1), ("prep", ctxs["prep"], 1), ("fused", ctxs["fused"], 4)):
+        for name, c, M in (("fused", ctxs["fused"], 1), ("prep", ctxs["prep"], 1), ("fused", ctxs["fused"], 4),
+                           ("dot4", ctxs["dot4"], 4)):
             say("majority outliers", kind, bits, N, K, M, name, pat)
             got = run_dense(c, torch, kind, bits, pk, sc, N, K, x[:M])
             e = max(relerr(got[m], ref14[m]) for m in range(M))
@@ -191,23 +193,25 @@ def test_dense_majority_outliers(torch_dev, oracle, monkeypatch, kind, bits, N, 
 
 
 @pytest.mark.parametrize("kind,bits", [(5, 0), (4, 3), (2, 0), (1, 0)])
-@pytest.mark.parametrize("M,env", [(4, {}), (8, {}), (32, {"BGL_NO_MFMA": 1})])
-def test_gemv_columns_outliers(torch_dev, oracle, monkeypatch, kind, bits, M, env):
-    """k_gemv over prepared digits: several columns, some with outliers, one plain."""
+@pytest.mark.parametrize("M,envs", [(4, [{}, {"BGL_NO_MFMA": 1}]), (8, [{}, {"BGL_NO_MFMA": 1}]), (32, [{"BGL_NO_MFMA": 1}])])
+def test_gemv_columns_outliers(torch_dev, oracle, monkeypatch, kind, bits, M, envs):
+    """k_gemv over prepared digits, and k_gemm_mfma: several columns, some with outliers, one plain."""
     torch = torch_dev
-    c = context(monkeypatch, **env)
+    ctxs = [(env, context(monkeypatch, **env)) for env in envs]
     N, K = 1536, 4096
     for i, pat in enumerate(PATTERNS[:3]):
-        say("gemv columns outliers", kind, bits, M, env, pat)
         x, wmul = outlier_case(pat, K, M, 300 + i)
         x[M - 1] = seeded_normal(301 + i, (K,))                    # a column without outliers
         pk, sc = make_weights(oracle, kind, bits, N, K, wmul, 310 + i)
-        got = run_dense(c, torch, kind, bits, pk, sc, N, K, x)
         ref = oracle.gemm_f32(kind, pk, sc, x, bits=bits)
-        for m in range(M):
-            e = relerr(got[m], ref[m])
-            assert e <= TOL, (pat, m, e)
-    c.close()
+        for env, c in ctxs:
+            say("gemv columns outliers", kind, bits, M, env, pat)
+            got = run_dense(c, torch, kind, bits, pk, sc, N, K, x)
+            for m in range(M):
+                e = relerr(got[m], ref[m])
+                assert e <= TOL, (pat, env, m, e)
+    for _, c in ctxs:
+        c.close()
 
 
 @pytest.mark.parametrize("kind,bits", [(5, 0), (2, 0), (4, 5), (1, 0)])
@@ -254,7 +258,7 @@ def nonfinite_weights(oracle, kind, bits, N, K, seed):
 
 
 @pytest.mark.parametrize("kind,bits", [(5, 0), (1, 0), (2, 0), (4, 2), (4, 9), (4, 15)])
-@pytest.mark.parametrize("M,env", [(1, {}), (1, {"BGL_X_FUSE": 0}), (1, {"BGL_NO_GEMV_X": 1}), (4, {}), (32, {}),
+@pytest.mark.parametrize("M,env", [(1, {}), (1, {"BGL_X_FUSE": 0}), (1, {"BGL_NO_GEMV_X": 1}), (4, {}), (4, {"BGL_NO_MFMA": 1}), (32, {}),
                                    (32, {"BGL_NO_MFMA": 1})])
 def test_nonfinite_activations(torch_dev, oracle, monkeypatch, kind, bits, M, env):
     torch = torch_dev
@@ -301,36 +305,34 @@ def run_moe(c, torch, gate, up, down, x, idx, w):
     return out.cpu().numpy()
 
 
-@pytest.mark.parametrize("env", [{}, {"BGL_NO_MOE_X": 1}])
-@pytest.mark.parametrize("T", [1, 8])
-def test_moe_outliers(torch_dev, oracle, monkeypatch, env, T):
+@pytest.mark.parametrize("T,envs", [(1, [{}, {"BGL_NO_MOE_X": 1}]), (8, [{}, {"BGL_NO_MFMA": 1}, {"BGL_NO_MOE_X": 1}])])
+def test_moe_outliers(torch_dev, oracle, monkeypatch, T, envs):
     """Routed FFN at DeepSeek-V2-Lite's expert shape (hidden 2048, expert 1408, top-6) over 12
     experts of mixed precision; token rows with outlier channels whose gate/up columns are small."""
     torch = torch_dev
-    c = context(monkeypatch, **env)
+    ctxs = [(env, context(monkeypatch, **env)) for env in envs]
     E, H, I, K = 12, 2048, 1408, 6
     fm = [(5, 0), (2, 0), (4, 7), (4, 12), (1, 0), (4, 15)]
     for i, pat in enumerate(["x1e4_w0.01", "x1e5_w0", "two_sizes_one_group"]):
-        say("moe outliers", env, T, pat)
         x, wmul = outlier_case(pat, H, T, 600 + i)
         gate, up, down = moe_descs(oracle, E, H, I, fm, 610 + 40 * i, wmul, np.ones(I, np.float32))
         idx, w = oracle.route(seeded_normal(620 + i, (T, E)), K, False)
-        got = run_moe(c, torch, gate, up, down, x, idx, w)
         ref = moe_ffn(oracle, gate, up, down, None, H, I, x, idx, w)
-        e = relerr(got, ref)
-        print(f"  max-rel {e:.3e}")
-        assert e <= TOL, (pat, e)
-    c.close()
+        for env, c in ctxs:
+            say("moe outliers", env, T, pat)
+            e = relerr(run_moe(c, torch, gate, up, down, x, idx, w), ref)
+            print(f"  max-rel {e:.3e}")
+            assert e <= TOL, (pat, env, e)
+    for _, c in ctxs:
+        c.close()
 
 
 def test_moe_majority_outliers(torch_dev, oracle, monkeypatch):
-    """The routed FFN at DeepSeek-V2-Lite's expert shape (k_moe_x, and k_moe_gemv over prepared
-    digits) with 33 or 40 of every group's 64 hidden channels at x1e2 .. x1e4 and zero gate/up
+    """The routed FFN at DeepSeek-V2-Lite's expert shape (k_moe_x, k_moe_gemv over prepared digits, and
+    k_moe_m) with 33 or 40 of every group's 64 hidden channels at x1e2 .. x1e4 and zero gate/up
     columns there, at T = 1 and 8.  The experts of a pattern are quantized once."""
     torch = torch_dev
-    cx = context(monkeypatch)
-    cg = context(monkeypatch, BGL_NO_MOE_X=1)
-    monkeypatch.delenv("BGL_NO_MOE_X", raising=False)
+    cx, cg, cm = context(monkeypatch, BGL_NO_MFMA=1), context(monkeypatch, BGL_NO_MOE_X=1), context(monkeypatch)
     E, H, I, K = 12, 2048, 1408, 6
     fm = [(5, 0), (2, 0), (4, 7), (4, 12), (1, 0), (4, 15)]
     for i, pat in enumerate(MAJORITY):
@@ -340,14 +342,14 @@ def test_moe_majority_outliers(torch_dev, oracle, monkeypatch):
             x = np.ascontiguousarray(x8[:T])
             idx, w = oracle.route(seeded_normal(860 + i + T, (T, E)), K, False)
             ref = moe_ffn(oracle, gate, up, down, None, H, I, x, idx, w)
-            for name, c in (("moe_x", cx), ("moe_gemv", cg)):
+            for name, c in (("moe_x", cx), ("moe_gemv", cg), ("moe_m", cm))[:3 if T > 1 else 2]:
                 say("moe majority outliers", name, T, pat)
                 got = run_moe(c, torch, gate, up, down, x, idx, w)
                 e = relerr(got, ref)
                 print(f"  max-rel {e:.3e}")
                 assert e <= TOL, (pat, name, T, e)
-    cx.close()
-    cg.close()
+    for c in (cx, cg, cm):
+        c.close()
 
 
 @pytest.mark.parametrize("env", [{}, {"BGL_NO_MOE_X": 1}])
@@ -372,32 +374,33 @@ def test_moe_nonfinite(torch_dev, oracle, monkeypatch, env):
     c.close()
 
 
-@pytest.mark.parametrize("T", [1, 8])
-def test_moe_outliers_mxfp4(torch_dev, oracle, monkeypatch, T):
+@pytest.mark.parametrize("T,envs", [(1, [{}]), (8, [{}, {"BGL_NO_MFMA": 1}])])
+def test_moe_outliers_mxfp4(torch_dev, oracle, monkeypatch, T, envs):
     """MXFP4 experts (beside int4 g32 and qNg64 ones) under the outlier patterns: their level-1 and
     non-finite cold paths (signed codes, no -8 correction) against the oracle's MXFP4 row."""
     torch = torch_dev
-    c = context(monkeypatch)
+    ctxs = [(env, context(monkeypatch, **env)) for env in envs]
     E, H, I, K = 8, 2048, 1408, 6
     fm = [(9, 4), (5, 0), (9, 4), (4, 12)]
     for i, pat in enumerate(["x1e4_w0.01", "x1e5_w0", "two_sizes_one_group"]):
-        say("moe outliers mxfp4", T, pat)
         x, wmul = outlier_case(pat, H, T, 640 + i)
         gate, up, down = moe_descs(oracle, E, H, I, fm, 650 + 40 * i, wmul, np.ones(I, np.float32))
         idx, w = oracle.route(seeded_normal(660 + i, (T, E)), K, False)
-        got = run_moe(c, torch, gate, up, down, x, idx, w)
         ref = moe_ffn(oracle, gate, up, down, None, H, I, x, idx, w)
-        e = relerr(got, ref)
-        print(f"  max-rel {e:.3e}")
-        assert e <= TOL, (pat, e)
+        for env, c in ctxs:
+            say("moe outliers mxfp4", T, env, pat)
+            e = relerr(run_moe(c, torch, gate, up, down, x, idx, w), ref)
+            print(f"  max-rel {e:.3e}")
+            assert e <= TOL, (pat, env, e)
     x = seeded_normal(670, (5, H))
     x[0, 10] = np.nan
     x[1, 300] = np.inf
     x[2, 7] = -np.inf
     gate, up, down = moe_descs(oracle, E, H, I, fm, 680, np.ones(H, np.float32), np.ones(I, np.float32))
     idx, w = oracle.route(seeded_normal(690, (5, E)), K, False)
-    got = run_moe(c, torch, gate, up, down, x, idx, w)
     ref = moe_ffn(oracle, gate, up, down, None, H, I, x, idx, w)
-    check_classes(got, ref, {})
-    assert np.all(np.isfinite(got[3:])) and relerr(got[3:], ref[3:]) <= TOL
-    c.close()
+    for env, c in ctxs:
+        got = run_moe(c, torch, gate, up, down, x, idx, w)
+        check_classes(got, ref, env)
+        assert np.all(np.isfinite(got[3:])) and relerr(got[3:], ref[3:]) <= TOL
+        c.close()
