@@ -206,14 +206,11 @@ def wbytes(kind, out, inn, bits):
     return alg_bytes(kind, out, inn, bits, 0)
 
 
-def shared_on_matrix_cores(kind, bits, T):
-    """Whether bgl_moe_layer_dev runs the shared experts as a dense block on the matrix cores (the
-    library's rule, bgl_moe.hip `shm`: >= BGL_MFMA_MIN_M = 16 tokens, BGL_NO_MFMA unset, and a kind
-    bgl_mfma_ok accepts: Q4G64, Q4G32H, Q8G64, or qNg64 with 2 <= n <= MF_MAXN = 10)."""
-    import beglin_amd
-    if T < 16 or os.environ.get("BGL_NO_MFMA", "0") not in ("", "0"):
-        return False
-    return kind in (beglin_amd.K_Q4G64, beglin_amd.K_Q4G32H, beglin_amd.K_Q8G64) or (kind == beglin_amd.K_QNG64 and 2 <= bits <= 10)
+def on_matrix_cores(T):
+    """Whether bgl_moe_layer_dev runs the whole layer on the matrix cores (k_moe_m): the library's rule (bgl_moe.hip
+    `moe_m_ok`) for a layer with shared experts and none in affine int4 or dense: from 3 tokens, no gather switch set."""
+    off = ("BGL_NO_MFMA", "BGL_NO_MOE_X", "BGL_FORCE_TR", "BGL_X_WAVES", "BGL_MOE_CAP")
+    return T >= 3 and all(os.environ.get(k, "0") in ("", "0") for k in off) and not os.environ.get("BGL_MOE_MERGE")
 
 
 class MoeWorkload:
@@ -231,7 +228,7 @@ class MoeWorkload:
         self.layers = []
         self.formats = []
         self.probe_sets = []          # per layer: the single tensors each gather launch streams
-        self.shm = []                 # per layer: the shared experts run on the matrix cores (not in the gathers)
+        self.mfma = on_matrix_cores(T)
         for _ in range(layers):
             fm = [CFG4_FORMATS[i] for i in rng.integers(0, len(CFG4_FORMATS), E)]
             shf = CFG4_FORMATS[int(rng.integers(0, len(CFG4_FORMATS)))]
@@ -262,13 +259,12 @@ class MoeWorkload:
             out = torch.empty((T, H), device="cuda")
             self.layers.append((stacks, tuple(sh), idx, w, out, nb, len(touched), rw))
             self.formats.append((fm, shf))
-            # the gather launches' tensors: routed gate+up (+ the shared gate+up, in the same launch
-            # below 16 tokens or where the shared experts stay in the gathers), routed down, shared down
+            # the gather launches' tensors: gate+up of routed and shared experts, then both down
+            # projections, in one launch on the matrix cores and in two elsewhere
             view = lambda hs: [beglin_amd.Tensor(hs[e]) for e in touched]
-            shm = shared_on_matrix_cores(shf[0], shf[1], T)
-            self.shm.append(shm)
-            gu = view(handles[0]) + view(handles[1])
-            sets = [gu, view(handles[2]), [sh[0], sh[1]], [sh[2]]] if shm else [gu + [sh[0], sh[1]], view(handles[2]), [sh[2]]]
+            gu = view(handles[0]) + view(handles[1]) + [sh[0], sh[1]]
+            down = view(handles[2])
+            sets = [gu, down + [sh[2]]] if self.mfma else [gu, down, [sh[2]]]
             self.probe_sets.append(sets)
 
     def run(self, tags=None):
@@ -351,9 +347,9 @@ KERNEL_SOURCES = {
     "cfg2": ("bgl_mlp_q.hip", "bgl_gemv.hip", "bgl_gemv_q.h", "bgl_gemv_impl.h", "bgl_device.h", "bgl_kernels.h"),
     "cfg1": ("bgl_gemv_x.hip", "bgl_gemv_x.h", "bgl_prep.hip", "bgl_device.h", "bgl_kernels.h"),
     "cfg3": ("bgl_gemv_x.hip", "bgl_gemv_x.h", "bgl_prep.hip", "bgl_device.h", "bgl_kernels.h"),
-    "cfg4": ("bgl_moe_x.hip", "bgl_moe_x.h", "bgl_moe.hip", "bgl_gemv_x.h", "bgl_prep.hip", "bgl_mfma.hip", "bgl_mlp.hip",
+    "cfg4": ("bgl_moe_x.hip", "bgl_moe_x.h", "bgl_moe_m.hip", "bgl_mfma_a.h", "bgl_moe.hip", "bgl_gemv_x.h", "bgl_gemv_impl.h",
              "bgl_device.h", "bgl_kernels.h"),
-    "cfg5": ("bgl_mfma.hip", "bgl_device.h", "bgl_kernels.h"),
+    "cfg5": ("bgl_mfma.hip", "bgl_mfma_a.h", "bgl_device.h", "bgl_kernels.h"),
 }
 
 
@@ -418,7 +414,7 @@ def moe_roofline(ctx, torch, stream, wl, reps):
     achieved = wl.nbytes() / (g_ms * 1e-3) / 1e9
     return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
-            "kernel": "k_moe_x / k_moe_x2 gathers (bgl_moe_x.h); from 16 tokens the shared experts' k_gemm_mfma (bgl_mfma.hip)",
+            "kernel": "k_moe_m (bgl_moe_m.hip)" if wl.mfma else "k_moe_x / k_moe_x2 gathers (bgl_moe_x.h)",
             "launches_per_step": g_n, "kernel_us_per_launch": round(g_ms * 1e3 / max(g_n, 1), 3),
             "bytes_per_launch": round(wl.nbytes() / max(g_n, 1)),
             "prep_us_per_step": round(p_ms * 1e3, 2), "prep_launches": p_n,
@@ -798,7 +794,7 @@ def main():
                               "how": "bgl_read_probe_dev over the touched experts' and the shared experts' tensors of "
                                      "each gather launch (launches of up to 64 tensors), 1024 x 256 threads, graph-timed; "
                                      "router weights and activations not read",
-                              "shared_on_matrix_cores_per_layer": [bool(v) for v in wl.shm]}
+                              "on_matrix_cores": wl.mfma}
         cpu = None if args.no_cpu else cpu_baseline_cfg4(wl, args.cpu_seconds, args.seed)
         finish(args, wl, ctx, graph, value, step_ms, wall, dtype, cfg, per_call, roof, cpu)
         return
