@@ -11,8 +11,8 @@
 // exact digits of the dot4 kernels held to 2^-23 of each 64-group's own maximum (2^-46 in groups of many
 // small elements), a column with such a group below 2^-14 of its maximum is multiplied a second time by
 // what the parts leave over (mf_wide, mf_leftover), so it is held to 2^-60.  (One test and the branch:
-// 28672 x 4096 at 5 columns 23.7 -> 24.0 us, 4096 x 4096 11.1 -> 11.4; a call with such a column takes
-// up to twice as long.)
+// 28672 x 4096 at 5 columns 23.4 -> 23.8 us, 4096 x 4096 at 5 and 15 11.1 -> 11.4 and 12.0 -> 12.3; a call
+// with such a column takes up to twice as long.)
 //
 // Layout.  A (weights, 16 rows x 32 k per instruction): lane l holds row l%16 and the 8 elements
 // 8*(l/16)..+7 of the 32-element K-step -- with the device's 16-byte chunk layout that is one
@@ -145,21 +145,13 @@ __device__ __forceinline__ float mf_leftover(float x, int sh) {
 template <int SPL>
 __device__ __forceinline__ bool mf_wide(const float4 (&v)[SPL][2], uint32_t lo, int n, int e) {
     const float thr = ldexpf(1.0f, e - 14);
-    if (!__any(__uint_as_float(lo) < thr)) return false;
+    const uint64_t low = __ballot(__uint_as_float(lo) < thr);
+    if (!low || !mf_three_lanes(low)) return false;                // (ordinary columns: one value in 5000 lies there)
     const int lane = threadIdx.x & 63;
     bool wide = false;
 #pragma unroll
     for (int j = 0; j < SPL; j++) {
         const bool in = lane + 64 * j < n;
-        auto below = [&](float x) { return in && fabsf(x) < thr; };
-        int cnt = 0;                                               // over the wave's 8 groups, zeros too
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const float4 q = v[j][h];
-            cnt += __popcll(__ballot(below(q.x))) + __popcll(__ballot(below(q.y))) + __popcll(__ballot(below(q.z))) +
-                   __popcll(__ballot(below(q.w)));
-        }
-        if (cnt < BGL_X_SMALL_MAX) continue;                       // (more small than large is 33 of 64, zeros among them)
         int c = 0;                                                 // small + 256 * large of the lane's 8, then of its group's 64
 #pragma unroll
         for (int h = 0; h < 2; h++) {

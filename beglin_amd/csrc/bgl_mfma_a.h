@@ -174,6 +174,15 @@ __device__ __forceinline__ void exch(const PRaw<FMT, NB> &p, ARaw<FMT, NB> (&a)[
     }
 }
 
+// Whether three of some byte's bits are set (scalar work).  Lanes 8g..8g+7 hold a 64-value group, 8 values
+// each: bgl_x_level1 wants 22 small ones (or 33 small and zero ones), so at least three of them hold one.
+__device__ __forceinline__ bool mf_three_lanes(uint64_t m) {
+    m -= (m >> 1) & 0x5555555555555555ull;
+    m = (m & 0x3333333333333333ull) + ((m >> 2) & 0x3333333333333333ull);
+    m = (m + (m >> 4)) & 0x0F0F0F0F0F0F0F0Full;
+    return ((m + 0x7D7D7D7D7D7D7D7Dull) & 0x8080808080808080ull) != 0;
+}
+
 __device__ __forceinline__ uint32_t sub_h2(uint32_t p, _Float16 c) {
     mf_h2 v = __builtin_bit_cast(mf_h2, p);
     const mf_h2 cc = {c, c};

@@ -114,7 +114,8 @@ __global__ __launch_bounds__(256) void k_moe_frag(MoeFrag F) {
     }
     bool wide = false;
     const float thr = ldexpf(1.0f, e - 14);
-    if (__any(__uint_as_float(lo) < thr))                 // (a group's 8 slots are 8 lanes, all of them or none in the row)
+    const uint64_t low = __ballot(__uint_as_float(lo) < thr);
+    if (low && mf_three_lanes(low))                       // (a group's 8 slots are 8 lanes, all of them or none in the row)
         for (int i = threadIdx.x, j = 0; i < n8; i += 256, j++) {
             float v8[8];
             slot(i, j, v8);
