@@ -3,8 +3,8 @@
 //
 // Numerics.  Weight codes are exact in fp16 (int4 and int8 codes, qNg64 codes for n <= 10), so
 // the decode is exact.  Each activation column is scaled by a power of two so its largest
-// magnitude lies in [2^13, 2^14), then split as hi = fp16(x') and lo = fp16(x' - hi), both rounded
-// toward zero (x' - hi is exact in fp32): hi + lo holds x' to about 2^-21 of the column maximum.  v_mfma_f32_16x16x32_f16 multiplies exactly and
+// magnitude lies in [2^13, 2^14), then split as hi = fp16(x') and lo = fp16(x' - hi), hi rounded
+// toward zero (x' - hi is exact in fp32) and lo to nearest: hi + lo holds x' to 2^-22 of itself.  v_mfma_f32_16x16x32_f16 multiplies exactly and
 // accumulates in fp32; each quantization group's partial sum is folded with its fp32 scale (one
 // FMA per output per group) and the column factor 2^-(14-e) is applied at the end.
 // The fp16 parts end at 2^-24, 2^-38 of the column's maximum over the split.  At 2..15 columns, which the
@@ -134,7 +134,7 @@ __device__ __forceinline__ float mf_leftover(float x, int sh) {
     const float v = ldexpf(x, sh);
     const mf_h2 h = __builtin_bit_cast(mf_h2, __builtin_amdgcn_cvt_pkrtz(v, 0.0f));
     const float r = v - (float)h[0];
-    const mf_h2 l = __builtin_bit_cast(mf_h2, __builtin_amdgcn_cvt_pkrtz(r, 0.0f));
+    const mf_h2 l = mf_cvt_rn(r, 0.0f);
     return r - (float)l[0];
 }
 
@@ -356,7 +356,8 @@ second_product:                                                    // level 1: a
             const float4 a = xv[ci][j][0], b = xv[ci][j][1];
             const float v8[8] = {a.x, a.z, a.y, a.w, b.x, b.z, b.y, b.w};   // element order {0,2,1,3,4,6,5,7}
             // hi = fp16(x') rounded toward zero, two at a time; x' - hi is exact in fp32 (hi is x'
-            // cut to 11 bits); lo = fp16 of that, toward zero
+            // cut to 11 bits); lo = fp16 of that, to nearest (toward zero its error would not cancel:
+            // 1.6e-7 of the product, see the numerics above)
             uint32_t H[4], Lo[4];
 #pragma unroll
             for (int k = 0; k < 4; k++) {
@@ -364,7 +365,7 @@ second_product:                                                    // level 1: a
                 const mf_h2 hh = __builtin_bit_cast(mf_h2, __builtin_amdgcn_cvt_pkrtz(v0, v1));
                 const float r0 = v0 - (float)hh[0], r1 = v1 - (float)hh[1];
                 const uint32_t hw = __builtin_bit_cast(uint32_t, hh);
-                const uint32_t lw = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(r0, r1));
+                const uint32_t lw = __builtin_bit_cast(uint32_t, mf_cvt_rn(r0, r1));
                 H[k] = ok ? hw : 0u;                               // K-steps past the split: zero fragments
                 Lo[k] = ok ? lw : 0u;
             }

@@ -174,6 +174,13 @@ __device__ __forceinline__ void exch(const PRaw<FMT, NB> &p, ARaw<FMT, NB> (&a)[
     }
 }
 
+// Two floats as halves to nearest, in one v_cvt_pk_f16_f32: the lo parts (the hi parts go toward zero).
+__device__ __forceinline__ mf_h2 mf_cvt_rn(float a, float b) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    const f2 v = {a, b};
+    return __builtin_convertvector(v, mf_h2);
+}
+
 // Whether three of some byte's bits are set (scalar work).  Lanes 8g..8g+7 hold a 64-value group, 8 values
 // each: bgl_x_level1 wants 22 small ones (or 33 small and zero ones), so at least three of them hold one.
 __device__ __forceinline__ bool mf_three_lanes(uint64_t m) {

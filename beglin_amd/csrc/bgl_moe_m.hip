@@ -36,7 +36,7 @@
 
 // ------------------------------------------------------------------ activation fragments
 // One workgroup per row: x' = x * 2^(14-e) (e: exponent of the row's largest finite |x|) as hi = fp16(x')
-// and lo = fp16(x' - hi), toward zero, in [row][K/32][hi: 32 halves | lo: 32 halves], eight values as
+// toward zero and lo = fp16(x' - hi) to nearest, in [row][K/32][hi: 32 halves | lo: 32 halves], eight values as
 // {0,2,1,3,4,6,5,7}; xe[row] = {e - 14, bit 0: the row holds NaN or +-Inf (as 0 here)}.
 // A row of a wide range (a 64-value group with as many elements below 2^(e-14) as bgl_x_level1 asks for: the
 // parts then hold less than exact digits under that group's own exponent would) also gets the parts of what
@@ -53,7 +53,7 @@ struct MoeFrag {
 __device__ __forceinline__ void mm_parts2(float &v0, float &v1, uint32_t &h, uint32_t &l) {
     const mf_h2 hh = __builtin_bit_cast(mf_h2, __builtin_amdgcn_cvt_pkrtz(v0, v1));
     v0 -= (float)hh[0]; v1 -= (float)hh[1];
-    const mf_h2 ll = __builtin_bit_cast(mf_h2, __builtin_amdgcn_cvt_pkrtz(v0, v1));
+    const mf_h2 ll = mf_cvt_rn(v0, v1);
     v0 -= (float)ll[0]; v1 -= (float)ll[1];
     h = __builtin_bit_cast(uint32_t, hh);
     l = __builtin_bit_cast(uint32_t, ll);
