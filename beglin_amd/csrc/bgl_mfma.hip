@@ -138,14 +138,13 @@ __device__ __forceinline__ float mf_leftover(float x, int sh) {
     return r - (float)l[0];
 }
 
-// Whether a wave's column (its slots in v, of which those below n are real; lo: the lane's smallest |x| bits,
+// Whether a wave's column (its slots in v, of which those below n are real; low: the lanes that hold a small one,
 // e: the exponent of the column's largest magnitude) has a 64-value group with as many small elements as
 // bgl_x_level1 asks for, small being below 2^(e-14).  In the other groups at most 21 elements lie that low
 // and at least as many above, so the digits, 2^-23 of their largest, were no finer than the fp16 parts.
 template <int SPL>
-__device__ __forceinline__ bool mf_wide(const float4 (&v)[SPL][2], uint32_t lo, int n, int e) {
+__device__ __forceinline__ bool mf_wide(const float4 (&v)[SPL][2], uint64_t low, int n, int e) {
     const float thr = ldexpf(1.0f, e - 14);
-    const uint64_t low = __ballot(__uint_as_float(lo) < thr);
     if (!low || !mf_three_lanes(low)) return false;                // (ordinary columns: one value in 5000 lies there)
     const int lane = threadIdx.x & 63;
     bool wide = false;
@@ -282,7 +281,7 @@ second_product:                                                    // level 1: a
     // their products code * scale * x one element at a time (IEEE propagation, as the reference's
     // fp32-product sums).
     int xe[CPW];                                                   // one column tile: the columns' exponents, and the
-    uint32_t xlo[CPW];                                             // lane's smallest |x| bits, for what follows the barrier
+    uint64_t xlow[CPW];                                            // lanes with small values, for what follows the barrier
 #pragma unroll
     for (int ci = 0; ci < CPW; ci++) {
         const int m = ci * NW + wave;
@@ -290,7 +289,7 @@ second_product:                                                    // level 1: a
         // the column's largest |x| bits over the split; Inf / NaN bits exceed every finite value's, so
         // only then (rare) are they zeroed and the maximum taken again
         uint32_t mb = 0u;
-        if constexpr (CT == 1) xlo[ci] = 0x7fffffffu;
+        uint32_t lo = 0x7fffffffu;                                 // one column tile: the lane's smallest |x| bits
 #pragma unroll
         for (int j = 0; j < SPL; j++)
 #pragma unroll
@@ -301,7 +300,7 @@ second_product:                                                    // level 1: a
                 const uint32_t t = max(max(a, b), max(c, d));
                 mb = m < L.M && lane + 64 * j < 4 * ns ? max(mb, t) : mb;
                 // (slots past the split are copies of the column's first)
-                if constexpr (CT == 1) xlo[ci] = min(min(min(a, b), min(c, d)), xlo[ci]);
+                if constexpr (CT == 1) lo = min(min(min(a, b), min(c, d)), lo);
             }
         mb = wave_max_u32(mb);
         if (lane == 0) cnf[m] = 0;
@@ -345,7 +344,8 @@ second_product:                                                    // level 1: a
                 sh = MF_RES_BITS;
                 use = use && cwd[m];                               // (this wave wrote it)
             }
-            xe[ci] = e;
+            xe[ci] = __builtin_amdgcn_readfirstlane(e);
+            xlow[ci] = __ballot(__uint_as_float(lo) < ldexpf(1.0f, e - 14));
         }
         const int ct = m >> 4, ml = m & 15;
 #pragma unroll
@@ -386,7 +386,7 @@ second_product:                                                    // level 1: a
 #pragma unroll
             for (int ci = 0; ci < CPW; ci++) {
                 const int m = ci * NW + wave;
-                const bool wide = m < L.M && mf_wide<SPL>(xv[ci], xlo[ci], 4 * ns, xe[ci]);
+                const bool wide = m < L.M && mf_wide<SPL>(xv[ci], xlow[ci], 4 * ns, xe[ci]);
                 if (lane == 0) cwd[m] = wide;
             }
         }
